@@ -4,10 +4,6 @@
 
 namespace qbg {
 
-#define QBG_F4(A, B)                                                          \
-  {A * B, A, B, f4::Launch<A, B>::L, &f4::Launch<A, B>::zbwd, &f4::Launch<A, B>::zfwd, \
-   &f4::Launch<A, B>::xpass, &f4::Launch<A, B>::ypass}
-
 static const F4Ops ops_d[] = {
     QBG_F4(18, 11),   // 198
     QBG_F4(15, 14),   // 210

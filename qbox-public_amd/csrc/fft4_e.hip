@@ -5,10 +5,6 @@
 
 namespace qbg {
 
-#define QBG_F4(A, B)                                                          \
-  {A * B, A, B, f4::Launch<A, B>::L, &f4::Launch<A, B>::zbwd, &f4::Launch<A, B>::zfwd, \
-   &f4::Launch<A, B>::xpass, &f4::Launch<A, B>::ypass}
-
 static const F4Ops ops_e[] = {
     QBG_F4(18, 5),    // 90
     QBG_F4(16, 6),    // 96

@@ -5,10 +5,6 @@
 
 namespace qbg {
 
-#define QBG_F4(A, B)                                                          \
-  {A * B, A, B, f4::Launch<A, B>::L, &f4::Launch<A, B>::zbwd, &f4::Launch<A, B>::zfwd, \
-   &f4::Launch<A, B>::xpass, &f4::Launch<A, B>::ypass}
-
 static const F4Ops ops_f[] = {
     QBG_F4(20, 8),    // 160
     QBG_F4(14, 12),   // 168

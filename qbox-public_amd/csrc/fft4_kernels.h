@@ -677,3 +677,8 @@ struct Launch {
 
 }  // namespace f4
 }  // namespace qbg
+
+// registry entry of the split n1 x n2 (fft4_reg.cpp)
+#define QBG_F4(A, B)                                                          \
+  {A * B, A, B, f4::Launch<A, B>::L, &f4::Launch<A, B>::zbwd, &f4::Launch<A, B>::zfwd, \
+   &f4::Launch<A, B>::xpass, &f4::Launch<A, B>::ypass}
