@@ -108,11 +108,13 @@ int gemm_syrk(const double* A, long lda, int N, long K, double alpha, double gam
 int gemm_nn_splitk(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
                    double* C, long ldc, double* work, size_t work_doubles, hipStream_t s,
                    const int* skip = nullptr);
+// NN (FP64) whose output columns may be columns of A, N <= gemm_nn_tile_p():
+// one block holds all N columns of its rows and reads them before it writes
+int gemm_nn_tile_p();
+void gemm_nn_inplace(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
+                     double* C, long ldc, hipStream_t s);
 // NN (FP64) with F upper triangular (F[m + n*ldf] = 0 for m > n), N x N:
 // C[k + n*ldc] = sum_{m <= n} A[k + m*lda] F[m + n*ldf]
-// output columns (p) of one tile of the NN product: a gemm_nn call with N <= this
-// runs one tile per group of rows, which reads its rows before it writes them
-int gemm_nn_tile_p();
 void gemm_nn_triu(const double* A, long lda, const double* F, long ldf, long K, int N, double* C,
                   long ldc, hipStream_t s);
 // NN: C[k + n*ldc] (+)= sum_m A[k + m*lda] F[m + n*ldf]  (K rows, N cols, M sum)

@@ -4,14 +4,32 @@
 // (syrk/syr/potrf/trsm, src/SlaterDet.cpp:487-520).
 //
 // One kernel shape serves every product: D[p][q] = sum_r P(r,p) Q(r,q) on a
-// 128x128 (p x q) tile per block of 256 threads (2x2 waves of 64x64, each a
-// 4x4 grid of 16x16 MFMA blocks), the reduction staged through LDS in
-// chunks of KC with the next chunk prefetched into registers.  P is read
-// along r (P(r,p) = P[r + p*ldp]); Q along r (TN form, Q[r + q*ldq]) or
-// along q (NN form, Q[q + r*ldq]).  q is the contiguous index of the
-// output, so the 16 lanes of an MFMA column group store 16 consecutive
-// elements.  The compute type is FP64 (v_mfma_f64_16x16x4f64) or FP32
-// (v_mfma_f32_16x16x4f32); operands are converted while they are staged.
+// (32 BI) x (32 BJ) tile per block of 256 threads: 2x2 waves, each a BI x BJ
+// grid of 16x16 MFMA blocks.  P is read along r (P(r,p) = P[r + p*ldp]); Q
+// along r (TN form, Q[r + q*ldq]) or along q (NN form, Q[q + r*ldq]).  q is
+// the contiguous index of the output, so the 16 lanes of an MFMA column group
+// store 16 consecutive elements.  The compute type is FP64
+// (v_mfma_f64_16x16x4f64) or FP32 (v_mfma_f32_16x16x4f32); operands are
+// converted while they are staged.
+//
+// What bounds it: the FP64 MFMA (64 cycles each; the loop without its loads,
+// stores and barriers runs at 74 TFLOP/s), and what stands between the products of two
+// chunks.  So that has to be short:
+//   - the reduction is staged in chunks of KC through two LDS stages with one
+//     barrier per chunk; the loads of the chunk after next are in registers
+//     meanwhile, and two blocks share a CU;
+//   - operands contiguous along r keep r contiguous in LDS and the MFMA step t
+//     of a chunk multiplies the elements r = 4 (lane/16) + t, so a lane's
+//     operands of two (FP64) or four (FP32) steps are one 16-byte LDS read, and
+//     the 16-byte global loads go to LDS unchanged (transposing stores had
+//     8-way bank conflicts here);
+//   - rows past the edge are loaded from the last row (their products are not
+//     stored), so only the last chunk and the last q tile test anything.
+// 512 bands x 1024 projectors x 461336 in FP64: TN 11.8 -> 8.4 ms (58 TFLOP/s),
+// NN 10.2 -> 7.9 ms (61 TFLOP/s).  Tried and slower or equal: a barrier in the middle of a
+// chunk with the next operands in registers (spills), wave priorities, 96-row
+// tiles.  The tile follows the extents (pick below): the projections
+// of 8 atoms on 16 bands (K = 11364) take 9 us where a 128 x 128 tile took 95.
 //
 // MFMA lane layouts on a 64-wide wave (16x16x4): lane l holds A[l%16][l/16]
 // and B[l/16][l%16]; accumulator e of lane l is D[4e + l/16][l%16] for f64
@@ -45,10 +63,24 @@ struct Mfma<float> {
   static __device__ __forceinline__ int row(int e, int lane) { return 4 * (lane >> 4) + e; }
 };
 
-constexpr int TP = 128;       // output tile rows (p)
-constexpr int TQ = 128;       // output tile columns (q)
+// two adjacent elements, at the alignment of one: the callers' arrays promise no more
+template <typename T>
+struct Pair2;
+template <>
+struct Pair2<double> {
+  typedef double v __attribute__((ext_vector_type(2), aligned(8)));
+};
+template <>
+struct Pair2<float> {
+  typedef float v __attribute__((ext_vector_type(2), aligned(4)));
+};
+
 constexpr int KC = 16;        // reduction chunk
-constexpr int PAD = 16;       // LDS row padding (elements)
+// LDS row of an operand with r contiguous: KC elements and 16 bytes, so that
+// eight rows' 16-byte reads fall on distinct banks
+template <typename TC>
+constexpr int RS = KC + 16 / (int)sizeof(TC);
+constexpr int QPAD = 4;       // row padding of the NN operand (q contiguous)
 
 struct GemmArgs {
   const void* P;
@@ -70,11 +102,16 @@ struct GemmArgs {
   int nblk;         // tiles x splits; the grid is that rounded up to 8
 };
 
-template <typename TPm, typename TQm, typename TC, bool QR, typename TO>
+template <typename TPm, typename TQm, typename TC, bool QR, typename TO, int BI, int BJ>
 __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g) {
   typedef Mfma<TC> MF;
-  __shared__ TC Ps[KC][TP + PAD];
-  __shared__ TC Qs[KC][TQ + PAD];
+  constexpr int TP = 32 * BI, TQ = 32 * BJ, R = RS<TC>;
+  // a lane's elements of one 16-byte LDS read
+  constexpr int NV = 16 / (int)sizeof(TC);
+  typedef TC vlds __attribute__((ext_vector_type(NV)));
+  typedef TC vst __attribute__((ext_vector_type(2)));
+  __shared__ __align__(16) TC Ps[2][TP * R];
+  __shared__ __align__(16) TC Qs[2][QR ? TQ * R : KC * (TQ + QPAD)];
   if (g.skip && *g.skip) return;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   // blocks are dealt to the 8 XCDs round robin: renumber so that runs of
@@ -97,77 +134,125 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g) {
   const long rb = (long)split * g.rper;
   long re = min(g.nr, rb + g.rper);
   if (g.tri == 2) re = min(re, (long)p0 + TP);
-  const TPm* __restrict__ Pp = (const TPm*)g.P;
-  const TQm* __restrict__ Qp = (const TQm*)g.Q;
-  TC pv[8], qv[8];
+  typedef typename Pair2<TPm>::v vp;
+  typedef typename Pair2<TQm>::v vq;
+  // this thread's rows of the operands read along r: elements sr, sr + 1 of
+  // the chunk, rows srow + 32 j
+  const int sr = 2 * (tid & 7), srow = tid >> 3;
+  const TPm* pp[BI];
+#pragma unroll
+  for (int j = 0; j < BI; j++)
+    pp[j] = (const TPm*)g.P + (long)min(p0 + srow + 32 * j, g.np - 1) * g.ldp + sr;
+  // the NN operand: elements nq0, nq0 + 1 of rows nr0 + (16 / BJ) j
+  const int nq0 = 2 * (tid % (16 * BJ)), nr0 = tid / (16 * BJ);
+  const bool qedge = !QR && q0 + TQ > g.nq;
+  const TQm* qp[BJ];
+#pragma unroll
+  for (int j = 0; j < BJ; j++)
+    qp[j] = QR ? (const TQm*)g.Q + (long)min(q0 + srow + 32 * j, g.nq - 1) * g.ldq + sr
+               : (const TQm*)g.Q + q0 + nq0 + (long)(nr0 + (16 / BJ) * j) * g.ldq;
+  vp pv[BI];
+  vq qv[BJ];
   auto load = [&](long r0) {
-    const long r = r0 + (tid & 15);
+    const bool full = r0 + KC <= re;
+    if (full) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      const int p = p0 + (tid >> 4) + 16 * j;
-      pv[j] = (p < g.np && r < re) ? (TC)Pp[r + (long)p * g.ldp] : TC(0);
+      for (int j = 0; j < BI; j++) pv[j] = *(const vp*)(pp[j] + r0);
+    } else {
+#pragma unroll
+      for (int j = 0; j < BI; j++) {
+        pv[j].x = r0 + sr < re ? pp[j][r0] : TPm(0);
+        pv[j].y = r0 + sr + 1 < re ? pp[j][r0 + 1] : TPm(0);
+      }
     }
     if (QR) {
+      if (full) {
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const int q = q0 + (tid >> 4) + 16 * j;
-        qv[j] = (q < g.nq && r < re) ? (TC)Qp[r + (long)q * g.ldq] : TC(0);
+        for (int j = 0; j < BJ; j++) qv[j] = *(const vq*)(qp[j] + r0);
+      } else {
+#pragma unroll
+        for (int j = 0; j < BJ; j++) {
+          qv[j].x = r0 + sr < re ? qp[j][r0] : TQm(0);
+          qv[j].y = r0 + sr + 1 < re ? qp[j][r0 + 1] : TQm(0);
+        }
       }
     } else {
-      const int q = q0 + (tid & 127);
+      if (full && !qedge) {
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const long rr = r0 + (tid >> 7) + 2 * j;
-        qv[j] = (q < g.nq && rr < re) ? (TC)Qp[q + rr * g.ldq] : TC(0);
+        for (int j = 0; j < BJ; j++) qv[j] = *(const vq*)(qp[j] + r0 * g.ldq);
+      } else {
+#pragma unroll
+        for (int j = 0; j < BJ; j++) {
+          const bool ok = r0 + nr0 + (16 / BJ) * j < re;
+          qv[j].x = ok && q0 + nq0 < g.nq ? qp[j][r0 * g.ldq] : TQm(0);
+          qv[j].y = ok && q0 + nq0 + 1 < g.nq ? qp[j][r0 * g.ldq + 1] : TQm(0);
+        }
       }
     }
   };
-  auto store = [&]() {
+  auto store = [&](int st) {
 #pragma unroll
-    for (int j = 0; j < 8; j++) Ps[tid & 15][(tid >> 4) + 16 * j] = pv[j];
-    if (QR) {
+    for (int j = 0; j < BI; j++)
+      *(vst*)&Ps[st][(srow + 32 * j) * R + sr] = vst{(TC)pv[j].x, (TC)pv[j].y};
 #pragma unroll
-      for (int j = 0; j < 8; j++) Qs[tid & 15][(tid >> 4) + 16 * j] = qv[j];
-    } else {
-#pragma unroll
-      for (int j = 0; j < 8; j++) Qs[(tid >> 7) + 2 * j][tid & 127] = qv[j];
-    }
+    for (int j = 0; j < BJ; j++)
+      *(vst*)&Qs[st][QR ? (srow + 32 * j) * R + sr
+                        : (nr0 + (16 / BJ) * j) * (TQ + QPAD) + nq0] =
+          vst{(TC)qv[j].x, (TC)qv[j].y};
   };
-  const int wp = (w & 1) * 64, wq = (w >> 1) * 64;
-  typename MF::acc acc[4][4];
+  const int wp = (w & 1) * 16 * BI, wq = (w >> 1) * 16 * BJ;
+  const int c = lane & 15, g4 = 4 * (lane >> 4);
+  typename MF::acc acc[BI][BJ];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < BI; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = typename MF::acc{0, 0, 0, 0};
-  if (rb < re) load(rb);
-  for (long r0 = rb; r0 < re; r0 += KC) {
-    store();
-    __syncthreads();
-    if (r0 + KC < re) load(r0 + KC);
+    for (int j = 0; j < BJ; j++) acc[i][j] = typename MF::acc{0, 0, 0, 0};
+  if (rb < re) {
+    load(rb);
+    store(0);
+    if (rb + KC < re) load(rb + KC);
+  }
+  __syncthreads();
+  int st = 0;
+  for (long r0 = rb; r0 < re; r0 += KC, st ^= 1) {
 #pragma unroll
-    for (int kk = 0; kk < KC; kk += 4) {
-      const int kr = kk + (lane >> 4), c = lane & 15;
-      TC a[4], bq[4];
+    for (int h = 0; h < 4; h += NV) {
+      vlds a[BI], bq[BJ];
 #pragma unroll
-      for (int i = 0; i < 4; i++) a[i] = Ps[kr][wp + 16 * i + c];
+      for (int i = 0; i < BI; i++)
+        a[i] = *(const vlds*)&Ps[st][(wp + 16 * i + c) * R + g4 + h];
 #pragma unroll
-      for (int j = 0; j < 4; j++) bq[j] = Qs[kr][wq + 16 * j + c];
+      for (int j = 0; j < BJ; j++) {
+        if (QR) {
+          bq[j] = *(const vlds*)&Qs[st][(wq + 16 * j + c) * R + g4 + h];
+        } else {
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+          for (int t = 0; t < NV; t++)
+            bq[j][t] = Qs[st][(g4 + h + t) * (TQ + QPAD) + wq + 16 * j + c];
+        }
+      }
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = MF::mma(a[i], bq[j], acc[i][j]);
+      for (int t = 0; t < NV; t++)
+#pragma unroll
+        for (int i = 0; i < BI; i++)
+#pragma unroll
+          for (int j = 0; j < BJ; j++) acc[i][j] = MF::mma(a[i][t], bq[j][t], acc[i][j]);
+    }
+    if (r0 + KC < re) {
+      store(st ^ 1);                       // last read one barrier ago
+      if (r0 + 2 * KC < re) load(r0 + 2 * KC);
     }
     __syncthreads();
   }
   TO* o = (TO*)g.out + (long)split * g.sstride;
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int i = 0; i < BI; i++)
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < BJ; j++)
 #pragma unroll
       for (int e = 0; e < 4; e++) {
         const int p = p0 + wp + 16 * i + MF::row(e, lane);
-        const int q = q0 + wq + 16 * j + (lane & 15);
+        const int q = q0 + wq + 16 * j + c;
         if (p < g.np && q < g.nq) {
           TO* d = o + q + (long)p * g.ldo;
           const TO v = (TO)acc[i][j][e];
@@ -176,7 +261,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g) {
       }
 }
 
-// out[q + p*ldo] = alpha * sum_s partial[s][p][q] + gamma * Q[q*ldq] * P[p*ldp]
+// out[q + p*ldo] = alpha * sum_s partial[s][p][q] + gamma * Q[q*ldq] * P[p*ldp].
+// A block sums 64 outputs: wave y takes the splits y, y + 4, ... (eight loads
+// in flight), and the four sums are added in that order.
 template <typename TQm, typename TPm>
 __global__ __launch_bounds__(256) void k_split_reduce(const double* __restrict__ partial, int S,
                                                       int nq, int np, double alpha, double gamma,
@@ -185,14 +272,21 @@ __global__ __launch_bounds__(256) void k_split_reduce(const double* __restrict__
                                                       double* __restrict__ out, long ldo,
                                                       int sym, const int* __restrict__ skip) {
   if (skip && *skip) return;
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  if (t >= (long)nq * np) return;
+  __shared__ double sums[4][64];
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+  const long t = (long)blockIdx.x * 64 + x, tot = (long)nq * np;
   const int q = (int)(t % nq), p = (int)(t / nq);
   // symmetric products hold only q >= p: the upper part mirrors it
   const long src = (sym && q < p) ? (long)q * nq + p : t;
   double s = 0.0;
-  for (int k = 0; k < S; k++) s += partial[(long)k * nq * np + src];
-  double v = alpha * s;
+  if (t < tot) {
+#pragma unroll 8
+    for (int k = y; k < S; k += 4) s += partial[(long)k * tot + src];
+  }
+  sums[y][x] = s;
+  __syncthreads();
+  if (y || t >= tot) return;
+  double v = alpha * ((sums[0][x] + sums[1][x]) + (sums[2][x] + sums[3][x]));
   if (gamma != 0.0) v += gamma * (double)Q[(long)q * ldq] * (double)P[(long)p * ldp];
   out[q + (long)p * ldo] = v;
 }
@@ -213,28 +307,77 @@ int cu_count() {
   return cache[dev];
 }
 
-// the split count in [ceil(smax/2), smax] whose ntile*S blocks spread most
-// evenly over the CUs (blocks / (cus * rounds)); the smaller on ties
-long even_split(long smax, int ntile) {
-  if (smax <= 1) return smax;
-  const long cus = cu_count();
-  long best = smax;
-  double eff = 0.0;
-  for (long S = (smax + 1) / 2; S <= smax; S++) {
-    const long b = S * ntile;
-    const double e = (double)b / (double)(cus * ((b + cus - 1) / cus));
-    if (e > eff + 1e-9) { eff = e; best = S; }
+// Tile (32 bi x 32 bj) and reduction splits of one product.
+struct Pick {
+  int bi, bj;
+  long S;
+};
+
+// cycles of a chunk's barrier and LDS latency that no MFMA covers: with one
+// block on a CU, and with two
+constexpr double CHUNK_ALONE = 700, CHUNK_SHARED = 200;
+constexpr double REDUCE_BYTES = 2000;    // bytes a cycle of the partials' store and sum
+
+// The pick with the fewest cycles of the busiest CU: (blocks per CU) x
+// (chunks) x (MFMA cycles of a wave's bi x bj blocks, 64 each in FP64, 32 in
+// FP32, and the chunk's fixed cost) + the traffic of the split partials.  It
+// makes the tiles follow ragged extents (131 bands: two 96-row tiles), and
+// small outputs use small tiles and many splits.  maxS: the most splits (1:
+// none); bjs: bit j allows bj = j; fixed bi, or 0; sym: square tiles, upper ones only.
+Pick pick(int np, int nq, long nr, long maxS, unsigned bjs, int bi_fixed, bool sym, int prec) {
+  const double cus = cu_count(), mf = prec == QBG_PREC_FP64 ? 256 : 128;
+  const long chunks = (nr + KC - 1) / KC;
+  Pick best{4, 4, 1};
+  double bt = 1e300;
+  for (int bi = 1; bi <= 4; bi++) {
+    if (bi_fixed && bi != bi_fixed) continue;
+    const long tp = (np + 32 * bi - 1) / (32 * bi);
+    for (int bj = 1; bj <= 4; bj++) {
+      if (!(bjs >> bj & 1) || (sym && bj != bi)) continue;
+      const long tq = (nq + 32 * bj - 1) / (32 * bj);
+      const long tiles = sym ? tp * (tp + 1) / 2 : tp * tq;
+      for (int k = 1; k <= 8; k++) {
+        long S = std::max<long>(1, (long)(k * cus) / tiles);
+        S = std::min(S, std::min(maxS, std::max<long>(1, chunks / 2)));
+        const double blocks = (double)tiles * S;
+        const double rounds = blocks < 16 * cus ? (double)(((long)blocks + (long)cus - 1) /
+                                                           (long)cus)
+                                                : blocks / cus;
+        const double chunk = bi * bj * mf + (rounds < 2 ? CHUNK_ALONE : CHUNK_SHARED);
+        double t = rounds * (double)((chunks + S - 1) / S) * chunk;
+        if (maxS > 1) t += (double)S * np * nq * 16.0 / REDUCE_BYTES;
+        if (t < bt) {
+          bt = t;
+          best = {bi, bj, S};
+        }
+        if (maxS <= 1) break;
+      }
+    }
   }
   return best;
 }
 
-template <typename TPm, typename TQm, typename TC, bool QR, typename TO>
-void launch_gemm(GemmArgs g, hipStream_t s) {
+template <typename TPm, typename TQm, typename TC, bool QR, typename TO, int BI, int BJ>
+void launch_tile(GemmArgs g, hipStream_t s) {
+  g.tp = (g.np + 32 * BI - 1) / (32 * BI);
+  g.tq = (g.nq + 32 * BJ - 1) / (32 * BJ);
   const int ntile = g.tri == 1 ? g.tp * (g.tp + 1) / 2 : g.tp * g.tq;
   g.nblk = ntile * (int)((g.nr + g.rper - 1) / g.rper);
   const unsigned grid = (unsigned)((g.nblk + 7) & ~7);
-  hipLaunchKernelGGL((k_gemm<TPm, TQm, TC, QR, TO>), dim3(grid), dim3(256), 0, s, g);
+  hipLaunchKernelGGL((k_gemm<TPm, TQm, TC, QR, TO, BI, BJ>), dim3(grid), dim3(256), 0, s, g);
 }
+
+template <typename TPm, typename TQm, typename TC, bool QR, typename TO>
+void launch_gemm(const GemmArgs& g, Pick k, hipStream_t s) {
+#define QBG_TILE(I, J) \
+  if (k.bi == I && k.bj == J) return launch_tile<TPm, TQm, TC, QR, TO, I, J>(g, s);
+#define QBG_TILES(I) QBG_TILE(I, 1) QBG_TILE(I, 2) QBG_TILE(I, 4)
+  QBG_TILES(1) QBG_TILES(2) QBG_TILES(3) QBG_TILES(4)
+  if constexpr (QR) { QBG_TILE(1, 3) QBG_TILE(2, 3) QBG_TILE(3, 3) QBG_TILE(4, 3) }
+#undef QBG_TILES
+#undef QBG_TILE
+}
+constexpr unsigned BJ_TN = 0x1e, BJ_NN = 0x16;   // compiled bj of the two forms
 
 // split-K TN product; partials in FP64, reduced in a fixed order.  sym: the
 // product is symmetric (A = B, M = N): only the lower tiles are formed.
@@ -243,91 +386,80 @@ int tn_splitk(const TQm* A, long lda, const double* B, long ldb, int M, int N, l
               double alpha, double gamma, double* out, long ldo, double* work,
               size_t work_doubles, int prec, int sym, hipStream_t s, const int* skip) {
   if (M <= 0 || N <= 0 || K <= 0) return -1;
+  if ((size_t)M * N > work_doubles || (sizeof(TQm) == 4 && prec == QBG_PREC_FP64)) return -1;
   GemmArgs g{};
   g.skip = skip;
   g.P = B; g.ldp = ldb; g.Q = A; g.ldq = lda;
   g.np = N; g.nq = M; g.nr = K;
-  g.tp = (N + TP - 1) / TP; g.tq = (M + TQ - 1) / TQ;
   g.pfast = 0;
   g.tri = sym ? 1 : 0;
-  const long ksteps = (K + KC - 1) / KC;
-  // tiles that do work: the upper triangle (q >= p) of a symmetric product
-  const int ntile = sym && g.tp == g.tq ? g.tp * (g.tp + 1) / 2 : g.tp * g.tq;
-  // about four blocks per CU; for large outputs the partial traffic is kept
-  // well below the operand traffic (small outputs split freely); at most 32
-  // splits for a general product (64 measured no faster on 512 x 512
-  // outputs); a symmetric product takes the count in [smax/2, smax] whose
-  // blocks spread most evenly over the CUs (ten 128-tiles at 512 bands: 51)
-  long S = std::max<long>(1, (1024 + ntile - 1) / ntile);
-  S = std::min<long>(S, std::max<long>(1, ksteps / 4));
-  if ((long)M * N > (1L << 20))
-    S = std::min<long>(S, std::max<long>(1, (long)((double)K * (M + N) / (4.0 * M * N))));
-  if (!sym) S = std::min<long>(S, 32);
-  while (S > 1 && (size_t)S * M * N > work_doubles) S--;
-  if ((size_t)S * M * N > work_doubles) return -1;
-  if (sym) S = even_split(S, ntile);
-  g.rper = ((ksteps + S - 1) / S) * KC;
-  S = (K + g.rper - 1) / g.rper;
+  const Pick k = pick(N, M, K, (long)(work_doubles / ((size_t)M * N)), BJ_TN, 0, sym != 0, prec);
+  const long chunks = (K + KC - 1) / KC;
+  g.rper = ((chunks + k.S - 1) / k.S) * KC;
+  const long S = (K + g.rper - 1) / g.rper;
   g.out = work; g.ldo = M; g.sstride = (long)M * N; g.accumulate = 0;
-  if (prec == QBG_PREC_FP64) launch_gemm<double, TQm, double, true, double>(g, s);
-  else launch_gemm<double, TQm, float, true, double>(g, s);
+  // FP32 operands come with FP32 products only
+  if constexpr (sizeof(TQm) == 8) {
+    if (prec == QBG_PREC_FP64) launch_gemm<double, TQm, double, true, double>(g, k, s);
+  }
+  if (prec != QBG_PREC_FP64) launch_gemm<double, TQm, float, true, double>(g, k, s);
   const long tot = (long)M * N;
-  hipLaunchKernelGGL((k_split_reduce<TQm, double>), dim3((unsigned)((tot + 255) / 256)),
+  hipLaunchKernelGGL((k_split_reduce<TQm, double>), dim3((unsigned)((tot + 63) / 64)),
                      dim3(256), 0, s, work, (int)S, M, N, alpha, gamma, A, lda, B, ldb, out, ldo,
                      sym, skip);
   return 0;
 }
 
+// one_p: a single p tile holds all N columns (N <= gemm_nn_tile_p()), so that
+// the block that read a row of A is the only one that writes it
 template <typename TQm, typename TO>
 void nn(const TQm* A, long lda, const double* F, long ldf, long K, int N, int M, TO* C, long ldc,
-        int accumulate, int prec, int tri, hipStream_t s, const int* skip) {
+        int accumulate, int prec, int tri, int one_p, hipStream_t s, const int* skip) {
   if (K <= 0 || N <= 0 || M <= 0) return;
   GemmArgs g{};
   g.skip = skip;
   g.P = F; g.ldp = ldf; g.Q = A; g.ldq = lda;
   g.np = N; g.nq = (int)K; g.nr = M;
-  g.tp = (N + TP - 1) / TP; g.tq = (int)((K + TQ - 1) / TQ);
   g.pfast = 1;
   g.tri = tri ? 2 : 0;
   g.rper = ((M + KC - 1) / KC) * KC;
   g.out = C; g.ldo = ldc; g.sstride = 0; g.accumulate = accumulate;
-  if (prec == QBG_PREC_FP64) launch_gemm<double, TQm, double, false, TO>(g, s);
-  else launch_gemm<double, TQm, float, false, TO>(g, s);
+  const Pick k = pick(N, (int)K, M, 1, BJ_NN, one_p ? (N + 31) / 32 : 0, false, prec);
+  if constexpr (sizeof(TQm) == 8 && sizeof(TO) == 8) {
+    if (prec == QBG_PREC_FP64) launch_gemm<double, TQm, double, false, TO>(g, k, s);
+  }
+  if (prec != QBG_PREC_FP64) launch_gemm<double, TQm, float, false, TO>(g, k, s);
 }
 
 }  // namespace
 
 // NN with the reduction (M) split over blocks, partials in work, for products
-// whose output has too few 128x128 tiles to fill the device:
+// whose output has too few tiles to fill the device:
 // C[k + n*ldc] = sum_m A[k + m*lda] F[m + n*ldf]
 int gemm_nn_splitk(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
                    double* C, long ldc, double* work, size_t work_doubles, hipStream_t s,
                    const int* skip) {
   if (K <= 0 || N <= 0 || M <= 0) return -1;
+  if ((size_t)K * N > work_doubles) return -1;
   GemmArgs g{};
   g.skip = skip;
   g.P = F; g.ldp = ldf; g.Q = A; g.ldq = lda;
   g.np = N; g.nq = (int)K; g.nr = M;
-  g.tp = (N + TP - 1) / TP; g.tq = (int)((K + TQ - 1) / TQ);
   g.pfast = 1;
   g.tri = 0;
-  const long msteps = (M + KC - 1) / KC;
-  const int ntile = g.tp * g.tq;
-  long S = std::max<long>(1, (1024 + ntile - 1) / ntile);
-  S = std::min<long>(S, std::max<long>(1, msteps / 4));
-  while (S > 1 && (size_t)S * K * N > work_doubles) S--;
-  if ((size_t)S * K * N > work_doubles) return -1;
-  g.rper = ((msteps + S - 1) / S) * KC;
-  S = (M + g.rper - 1) / g.rper;
+  const long chunks = (M + KC - 1) / KC;
+  const Pick k = pick(N, (int)K, M, (long)(work_doubles / ((size_t)K * N)), BJ_NN, 0, false,
+                      QBG_PREC_FP64);
+  g.rper = ((chunks + k.S - 1) / k.S) * KC;
+  const long S = (M + g.rper - 1) / g.rper;
   g.out = work; g.ldo = K; g.sstride = K * N; g.accumulate = 0;
-  launch_gemm<double, double, double, false, double>(g, s);
+  launch_gemm<double, double, double, false, double>(g, k, s);
   const long tot = K * N;
-  hipLaunchKernelGGL((k_split_reduce<double, double>), dim3((unsigned)((tot + 255) / 256)),
+  hipLaunchKernelGGL((k_split_reduce<double, double>), dim3((unsigned)((tot + 63) / 64)),
                      dim3(256), 0, s, work, (int)S, (int)K, N, 1.0, 0.0, A, lda, F, ldf, C, ldc,
                      0, skip);
   return 0;
 }
-
 int gemm_tn_splitk(const double* A, long lda, const double* B, long ldb, int M, int N, long K,
                    double alpha, double gamma, double* out, long ldo, double* work,
                    size_t work_doubles, int prec, hipStream_t s, const int* skip) {
@@ -345,22 +477,26 @@ int gemm_syrk(const double* A, long lda, int N, long K, double alpha, double gam
   return tn_splitk(A, lda, A, lda, N, N, K, alpha, gamma, out, ldo, work, work_doubles,
                    QBG_PREC_FP64, 1, s, skip);
 }
-int gemm_nn_tile_p() { return TP; }
+int gemm_nn_tile_p() { return 128; }
 void gemm_nn_triu(const double* A, long lda, const double* F, long ldf, long K, int N, double* C,
                   long ldc, hipStream_t s) {
-  nn(A, lda, F, ldf, K, N, N, C, ldc, 0, QBG_PREC_FP64, 1, s, nullptr);
+  nn(A, lda, F, ldf, K, N, N, C, ldc, 0, QBG_PREC_FP64, 1, 0, s, nullptr);
+}
+void gemm_nn_inplace(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
+                     double* C, long ldc, hipStream_t s) {
+  nn(A, lda, F, ldf, K, N, M, C, ldc, 0, QBG_PREC_FP64, 0, 1, s, nullptr);
 }
 void gemm_nn(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
              double* C, long ldc, int accumulate, int prec, hipStream_t s, const int* skip) {
-  nn(A, lda, F, ldf, K, N, M, C, ldc, accumulate, prec, 0, s, skip);
+  nn(A, lda, F, ldf, K, N, M, C, ldc, accumulate, prec, 0, 0, s, skip);
 }
 void gemm_nn(const float* A, long lda, const double* F, long ldf, long K, int N, int M,
              double* C, long ldc, int accumulate, int prec, hipStream_t s) {
-  nn(A, lda, F, ldf, K, N, M, C, ldc, accumulate, prec, 0, s, nullptr);
+  nn(A, lda, F, ldf, K, N, M, C, ldc, accumulate, prec, 0, 0, s, nullptr);
 }
 void gemm_nn(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
              float* C, long ldc, int accumulate, int prec, hipStream_t s) {
-  nn(A, lda, F, ldf, K, N, M, C, ldc, accumulate, prec, 0, s, nullptr);
+  nn(A, lda, F, ldf, K, N, M, C, ldc, accumulate, prec, 0, 0, s, nullptr);
 }
 
 // ------------------------------------------------------- Cholesky, inverse
@@ -550,7 +686,7 @@ static void potrf_blocked(double* S, int n, int lds, int* info, double* ws, hipS
                        info, ws);
     // A22 += L21 (-L21^T)
     nn(S + (j0 + jb) + (long)j0 * lds, lds, ws, CB, rows, rows, jb, S + (j0 + jb) +
-       (long)(j0 + jb) * lds, lds, 1, QBG_PREC_FP64, 0, s, info);
+       (long)(j0 + jb) * lds, lds, 1, QBG_PREC_FP64, 0, 0, s, info);
   }
 }
 

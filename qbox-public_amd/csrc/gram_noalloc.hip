@@ -8,8 +8,8 @@
 // device address comes from hipGetSymbolAddress, once per device with that
 // device current; kernels only ever see that address.
 //
-// The update C <- C L^-T runs in place, one column block of at most GEMM_TP
-// columns per launch from the last block to the first: block J of the result
+// The update C <- C L^-T runs in place, one column block of at most
+// gemm_nn_tile_p() columns per launch from the last block to the first: block J of the result
 // needs the old columns [0, j1) only, the columns left of J are still old
 // when J runs, and within a launch each output tile is written after its
 // whole reduction, by the one work-group that read those rows.  So no copy
@@ -97,8 +97,8 @@ int qbg_gram_noalloc(qbg_ctx* c, double* cc, int ldc, int ngw, int nst, int prec
     const int tp = qbg::gemm_nn_tile_p();
     for (int j0 = ((nst - 1) / tp) * tp; j0 >= 0; j0 -= tp) {
       const int j1 = std::min(nst, j0 + tp);
-      qbg::gemm_nn(cc, lda, X + (size_t)j0 * nst, nst, K, j1 - j0, j1, cc + (size_t)j0 * lda,
-                   lda, 0, QBG_PREC_FP64, s, nullptr);
+      qbg::gemm_nn_inplace(cc, lda, X + (size_t)j0 * nst, nst, K, j1 - j0, j1,
+                           cc + (size_t)j0 * lda, lda, s);
     }
     c->prof_end();
     QBG_HIP(c, hipStreamSynchronize(s));
