@@ -5,9 +5,9 @@
 namespace qbg {
 
 static const F4Ops ops_c[] = {
-    QBG_F4(16, 9),   // 144
-    QBG_F4(16, 10),   // 160
-    QBG_F4(21, 8),   // 168
+    QBG_F4(12, 12),   // 144
+    QBG_F4(10, 16),   // 160
+    QBG_F4(14, 12),   // 168
 };
 
 const F4Ops* f4_table_c(int* count) {

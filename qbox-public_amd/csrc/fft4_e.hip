@@ -6,12 +6,12 @@
 namespace qbg {
 
 static const F4Ops ops_e[] = {
-    QBG_F4(18, 5),    // 90
-    QBG_F4(16, 6),    // 96
+    QBG_F4(9, 10),    // 90
+    QBG_F4(12, 8),    // 96
     QBG_F4(14, 8),    // 112
-    QBG_F4(18, 7),    // 126
-    QBG_F4(32, 4),    // 128
-    QBG_F4(12, 12),   // 144
+    QBG_F4(9, 14),    // 126
+    QBG_F4(8, 16),    // 128
+    QBG_F4(16, 9),    // 144
 };
 
 const F4Ops* f4_table_e(int* count) {

@@ -6,11 +6,11 @@
 namespace qbg {
 
 static const F4Ops ops_f[] = {
-    QBG_F4(20, 8),    // 160
-    QBG_F4(14, 12),   // 168
-    QBG_F4(22, 9),    // 198
+    QBG_F4(16, 10),   // 160
+    QBG_F4(12, 14),   // 168
+    QBG_F4(11, 18),   // 198
     QBG_F4(14, 15),   // 210
-    QBG_F4(32, 7),    // 224
+    QBG_F4(14, 16),   // 224
 };
 
 const F4Ops* f4_table_f(int* count) {

@@ -14,7 +14,7 @@ static const F4Ops ops_g[] = {
     QBG_F4(8, 5),   // 40
     QBG_F4(7, 6),   // 42
     QBG_F4(11, 4),   // 44
-    QBG_F4(16, 3),   // 48
+    QBG_F4(12, 4),   // 48
 };
 
 const F4Ops* f4_table_g(int* count) {

@@ -10,7 +10,7 @@ static const F4Ops ops_h[] = {
     QBG_F4(11, 6),   // 66
     QBG_F4(10, 7),   // 70
     QBG_F4(9, 8),   // 72
-    QBG_F4(20, 4),   // 80
+    QBG_F4(10, 8),   // 80
     QBG_F4(12, 7),   // 84
 };
 

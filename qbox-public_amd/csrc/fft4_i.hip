@@ -9,7 +9,7 @@ static const F4Ops ops_i[] = {
     QBG_F4(11, 10),   // 110
     QBG_F4(15, 8),   // 120
     QBG_F4(12, 11),   // 132
-    QBG_F4(20, 7),   // 140
+    QBG_F4(14, 10),   // 140
 };
 
 const F4Ops* f4_table_i(int* count) {

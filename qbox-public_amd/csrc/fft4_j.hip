@@ -7,7 +7,7 @@ namespace qbg {
 static const F4Ops ops_j[] = {
     QBG_F4(14, 11),   // 154
     QBG_F4(16, 11),   // 176
-    QBG_F4(20, 9),   // 180
+    QBG_F4(15, 12),   // 180
     QBG_F4(16, 12),   // 192
 };
 

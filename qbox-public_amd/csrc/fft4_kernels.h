@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void kz_bwd(const double* __restrict__ c, long
     if constexpr (!Mp::pfa) {
 #pragma unroll
       for (int k1 = 1; k1 < N1; k1++)
-        if (q) a[k1] = mul(a[k1], twl<T, +1>(tw, q * k1));
+        a[k1] = mul(a[k1], twl<T, +1>(tw, q * k1));
     }
   }
   __syncthreads();                        // the prime-factor reads cross threads
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(256) void kz_fwd(const cpx<T>* __restrict__ zbuf,
     if constexpr (!Mp::pfa) {
 #pragma unroll
       for (int m1 = 1; m1 < N2; m1++)
-        if (q) b[m1] = mul(b[m1], twl<T, -1>(tw, q * m1));
+        b[m1] = mul(b[m1], twl<T, -1>(tw, q * m1));
     }
   }
   __syncthreads();
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(xthreads(N1, N2)) void kx_bwd(
     if constexpr (!Mp::pfa) {
 #pragma unroll
       for (int k1 = 1; k1 < N1; k1++)
-        if (p) a[k1] = mul(a[k1], twl<T, +1>(tw, p * k1));
+        a[k1] = mul(a[k1], twl<T, +1>(tw, p * k1));
     }
 #pragma unroll
     for (int k1 = 0; k1 < N1; k1++) ex[kk * NP + k1 * N2 + p] = a[k1];
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(xthreads(N1, N2)) void kx_fwd(
     if constexpr (!Mp::pfa) {
 #pragma unroll
       for (int m1 = 1; m1 < N2; m1++)
-        if (p) b[m1] = mul(b[m1], twl<T, -1>(tw, p * m1));
+        b[m1] = mul(b[m1], twl<T, -1>(tw, p * m1));
     }
   }
   __syncthreads();
@@ -467,7 +467,7 @@ __global__ __launch_bounds__(xthreads(N1, N2)) void ky(
         if constexpr (!Mp::pfa) {
 #pragma unroll
           for (int m1 = 1; m1 < N2; m1++)
-            if (q) b[m1] = mul(b[m1], twl<T, -1>(tw, q * m1));
+            b[m1] = mul(b[m1], twl<T, -1>(tw, q * m1));
         }
       }
 #pragma unroll
@@ -499,21 +499,31 @@ __global__ __launch_bounds__(xthreads(N1, N2)) void ky(
   }
   const int p0 = blockIdx.z * PPB;
   const int p1 = min(nbatch, p0 + PPB);
+  // FP32 density: the rows of a pair are loaded while the pair before it is
+  // transformed (104 -> 87 us on a 96 x 110 x 120 grid, 75 bands).  The potential
+  // multiply and FP64 lost more to the registers than they gained.
+  constexpr bool AHEAD = MC == 1 && sizeof(T) == 4;
+  cpx<T> a[N1];
+  auto load_rows = [&](int pair) {
+    const auto xr = buf_res(run0 + pair * pstride, runbytes);
+#pragma unroll
+    for (int n1 = 0; n1 < N1; n1++) a[n1] = buf_load<T>(xr, jq[n1] + lo);
+  };
+  if (AHEAD && vA && p0 < p1) load_rows(p0);
   for (int pair = p0; pair < p1; pair++) {
     __syncthreads();                      // previous pair's readers of ex are done
     const auto xr = buf_res(run0 + pair * pstride, runbytes);
     if (vA) {                             // phase A, q = n2 (bwd)
-      cpx<T> a[N1];
-#pragma unroll
-      for (int n1 = 0; n1 < N1; n1++) a[n1] = buf_load<T>(xr, jq[n1] + lo);
+      if (!AHEAD) load_rows(pair);
       rdft<T, N1, +1>(a);
       if constexpr (!Mp::pfa) {
 #pragma unroll
         for (int k1 = 1; k1 < N1; k1++)
-          if (q) a[k1] = mul(a[k1], twl<T, +1>(tw, q * k1));
+          a[k1] = mul(a[k1], twl<T, +1>(tw, q * k1));
       }
 #pragma unroll
       for (int k1 = 0; k1 < N1; k1++) ex[xi * NP + k1 * N2 + q] = a[k1];
+      if (AHEAD && pair + 1 < p1) load_rows(pair + 1);
     }
     __syncthreads();
     cpx<T> b[N2];
@@ -531,7 +541,7 @@ __global__ __launch_bounds__(xthreads(N1, N2)) void ky(
         if constexpr (!Mp::pfa) {
 #pragma unroll
           for (int m1 = 1; m1 < N2; m1++)
-            if (q) b[m1] = mul(b[m1], twl<T, -1>(tw, q * m1));
+            b[m1] = mul(b[m1], twl<T, -1>(tw, q * m1));
         }
       }
       __syncthreads();
@@ -553,8 +563,10 @@ __global__ __launch_bounds__(xthreads(N1, N2)) void ky(
         const double f1 = fac[2 * pair], f2 = fac[2 * pair + 1];
 #pragma unroll
         for (int k2 = 0; k2 < N2; k2++) {
+          // four FP64 instructions a point
           const double p1v = (double)b[k2].x, p2v = (double)b[k2].y;
-          acc[k2 % NACC] += f1 * p1v * p1v + f2 * p2v * p2v;
+          acc[k2 % NACC] += f1 * (p1v * p1v);
+          acc[k2 % NACC] += f2 * (p2v * p2v);
         }
       }
     } else if (mode == Y_BWD_FULL) {

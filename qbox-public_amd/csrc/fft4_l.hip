@@ -6,7 +6,7 @@ namespace qbg {
 
 static const F4Ops ops_l[] = {
     QBG_F4(16, 16),   // 256
-    QBG_F4(24, 11),   // 264
+    QBG_F4(22, 12),   // 264
     QBG_F4(20, 14),   // 280
 };
 

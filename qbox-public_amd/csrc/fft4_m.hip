@@ -5,8 +5,8 @@
 namespace qbg {
 
 static const F4Ops ops_m[] = {
-    QBG_F4(24, 12),   // 288
-    QBG_F4(28, 11),   // 308
+    QBG_F4(18, 16),   // 288
+    QBG_F4(22, 14),   // 308
     QBG_F4(20, 16),   // 320
 };
 

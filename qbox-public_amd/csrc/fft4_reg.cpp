@@ -11,10 +11,15 @@
 // compile-time constants and load only the active rows: 47 bands with two spins
 // in a 15 x 17.5 x 21 bohr cell (45 Ry, FP32) evaluate in 0.61 ms where the
 // Stockham passes take 1.27 ms, 64 bands at three k-points (55 Ry, 15.5 bohr)
-// in 2.00 ms where they take 5.66 ms.  The split of a length in fft4_g..o is the
-// one with the fewest wave instructions (DFT operations of the two phases
-// times the waves that run them, plus twiddles where n1 and n2 share a
-// factor), with factors above 24 left out for their register use.
+// in 2.00 ms where they take 5.66 ms.
+//
+// Which split: the one whose passes are fastest with every divisor pair timed
+// (cubes of 36 to 256, 32 to 128 bands, both precisions).  Two balanced factors of at most
+// 16 win everywhere, coprime or not: 80 as 10 x 8 takes 0.60 of the time of
+// 20 x 4, 168 as 14 x 12 0.82 of 21 x 8, 180 as 15 x 12 0.81 of 20 x 9.
+// A factor above 16 needs more than four waves a block, fewer blocks fit, and the
+// long DFT is left to few of the waves; 198, 220, 252 and the lengths above 256
+// have no other.
 #include "internal.h"
 
 namespace qbg {
