@@ -652,7 +652,7 @@ static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, do
     e->partial_doubles = std::max<size_t>(e->partial_doubles, ((size_t)e->M * nst + 255) / 256 + 16);
     e->partial_doubles = std::max<size_t>(e->partial_doubles,
                                           (size_t)((ngwm + 255) / 256) * ((nst + 31) / 32) * 8);
-    e->partial_doubles = std::max<size_t>(e->partial_doubles, (size_t)nsp * 64 * 6 + 16);
+    e->partial_doubles = std::max<size_t>(e->partial_doubles, (size_t)nsp * NLS_CHUNKS_MAX * 6);
     // split-K partials of the fnl product: up to 40 splits of M x nst
     e->work_doubles = std::max<size_t>((size_t)1 << 22, (size_t)40 * e->M * nst);
     // occupations times the weight of k-point 0 (of a set; 1 otherwise)
@@ -1195,12 +1195,12 @@ static int nl_mfma(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
       if (f32)
         launch_nl_stress_y((const float*)Y, K, ngw, e->d_gxw, e->d_tau, e->nsp, e->d_sp_first,
                            e->d_sp_npr, e->d_dt_off, e->d_dtwnl, e->d_a_m0, e->d_a_stride,
-                           e->d_m_l, e->d_partial, 64, e->o_nls, s,
+                           e->d_m_l, e->d_partial, e->o_nls, s,
                            e->cplx ? 2 : 1, e->Mh);
       else
         launch_nl_stress_y((const double*)Y, K, ngw, e->d_gxw, e->d_tau, e->nsp, e->d_sp_first,
                            e->d_sp_npr, e->d_dt_off, e->d_dtwnl, e->d_a_m0, e->d_a_stride,
-                           e->d_m_l, e->d_partial, 64, e->o_nls, s,
+                           e->d_m_l, e->d_partial, e->o_nls, s,
                            e->cplx ? 2 : 1, e->Mh);
     }
     ctx->prof_end();
@@ -1408,7 +1408,7 @@ static int nl_bf16(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
     if (compute_stress)
       launch_nl_stress_y((const float*)e->b_y32, Kp, ngw, e->d_gxw, e->d_tau, e->nsp,
                          e->d_sp_first, e->d_sp_npr, e->d_dt_off, e->d_dtwnl, e->d_a_m0,
-                         e->d_a_stride, e->d_m_l, e->d_partial, 64, e->o_nls, s,
+                         e->d_a_stride, e->d_m_l, e->d_partial, e->o_nls, s,
                          e->cplx ? 2 : 1, e->Mh);
     ctx->prof_end();
   }
@@ -1589,7 +1589,7 @@ static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, doub
     ctx->prof_begin(QBG_K_OTHER);
     const int nchunk = 64;
     launch_local_forces(e->d_idxv, e->vb.size, e->d_sftab, e->krange, e->kmin, e->d_lfgrp,
-                        e->nlfgrp, e->nsp, e->d_vps, e->d_rhops, e->d_g2iv, e->d_gxv, e->d_rhogt,
+                        e->nlfgrp, e->nsp, e->d_vps, e->d_rhops, e->d_g2iv, e->d_b, e->d_rhogt,
                         e->d_rhoelg, e->core ? e->d_vxcg : nullptr, e->d_rhoc, e->omega,
                         e->d_fesr, e->nat, e->d_vtemp, e->d_partial, nchunk, e->d_fion, s);
     ctx->prof_end();

@@ -35,12 +35,13 @@ void launch_sfac(const int32_t* idx, int ngv, const double* tab, int krange, con
                  const double* rhops, double* sfac, double* vion, double* dvion, double* rhopst,
                  hipStream_t s);
 // local forces; grp[3*g + {0,1,2}] = first atom, atoms (<= the group size),
-// species of group g; vt holds 2*nsp*ngv doubles
+// species of group g; vt holds 2*nsp*ngv doubles; b[3*axis + j] the
+// reciprocal vectors
 int local_forces_group_size(int krange);
 void launch_local_forces(const int32_t* idx, int ngv, const double* tab, int krange,
                          const int* kmin, const int32_t* grp, int ngrp, int nsp,
                          const double* vps, const double* rhops, const double* g2i,
-                         const double* gx, const double* rhogt, const double* rhoelg,
+                         const double* b, const double* rhogt, const double* rhoelg,
                          const double* vxcg, const double* rhoc, double omega, const double* fesr, int nat, double* vt, double* partial,
                          int nchunk, double* fion, hipStream_t s);
 // anl columns of every atom's projectors (FP64 if prec == 0, else FP32)
@@ -76,12 +77,14 @@ void launch_nl_forces_y(const T* A, const T* Y, long lda, int ngw, const double*
                         const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
                         int nat, double* partial, int nchunk, double* fion, hipStream_t s);
 
+// partial of launch_nl_stress_y: 6 nsp NLS_CHUNKS_MAX doubles
+constexpr int NLS_CHUNKS_MAX = 1024;
 template <typename T>
 void launch_nl_stress_y(const T* Y, long lda, int ngw, const double* gx, const double* tau,
                         int nsp, const int32_t* sp_first, const int32_t* sp_npr,
                         const int64_t* dt_off, const double* dtwnl, const int32_t* a_m0,
                         const int32_t* a_stride, const int32_t* m_l, double* partial,
-                        int nchunk, double* out6, hipStream_t s, int halves = 1, long mhalf = 0);
+                        double* out6, hipStream_t s, int halves = 1, long mhalf = 0);
 void launch_hart_ps_stress(const double* rhogt, const double* sfac, const double* rhops,
                            const double* g2i, const double* gx, int ngv, int nsp,
                            const double* fac2, const double* vxcg, const double* drhoc,

@@ -28,10 +28,10 @@ __device__ __forceinline__ void block_reduce_store(double (&v)[NV], double* __re
   if (threadIdx.x < NV) out[threadIdx.x] = red[threadIdx.x][0];
 }
 
-// the same sums through wave shuffles, then the 4 wave totals in order
-template <int NV>
+// the same sums through wave shuffles, then the NW wave totals in order
+template <int NV, int NW>
 __device__ __forceinline__ void block_reduce_shfl(double (&v)[NV], double* __restrict__ out) {
-  __shared__ double red[NV][4];
+  __shared__ double red[NV][NW];
 #pragma unroll
   for (int q = 0; q < NV; q++)
 #pragma unroll
@@ -44,7 +44,10 @@ __device__ __forceinline__ void block_reduce_shfl(double (&v)[NV], double* __res
   __syncthreads();
   if (threadIdx.x < NV) {
     const int q = threadIdx.x;
-    out[q] = ((red[q][0] + red[q][1]) + red[q][2]) + red[q][3];
+    double s = red[q][0];
+#pragma unroll
+    for (int k = 1; k < NW; k++) s += red[q][k];
+    out[q] = s;
   }
 }
 
@@ -363,8 +366,9 @@ __device__ __forceinline__ void eigr_from_tables(const double* __restrict__ tab,
   const double* p1 = tab + ((long)(a * 3 + 1) * krange + ky) * 2;
   const double* p2 = tab + ((long)(a * 3 + 2) * krange + kz) * 2;
   const double ca = p0[0], sa = p0[1], cb = p1[0], sb = p1[1], cc = p2[0], sc = p2[1];
-  re = ca * cb * cc - sa * sb * cc - sa * cb * sc - ca * sb * sc;
-  im = sa * sb * sc - sa * cb * cc - ca * sb * cc - ca * cb * sc;
+  const double x = ca * cb - sa * sb, y = ca * sb + sa * cb;
+  re = x * cc - y * sc;
+  im = -(x * sc + y * cc);
 }
 
 // sfac[is][ig] = sum_{a in is} exp(-iG.tau_a); then (src/EnergyFunctional.cpp:1085-1095)
@@ -460,7 +464,14 @@ void launch_core_dxc(int ngv, const double* vxcg, const double* rhocg, double* p
 // vtemp_s is formed once per species; a block then takes a chunk of G and a
 // group of up to LF_AG atoms of one species, with the atoms' per-axis phase
 // tables in LDS, so the G data is read once per group instead of per atom.
+// The sums run over the indices k of G = k0 b0 + k1 b1 + k2 b2 (28 bytes read a
+// vector with vtemp, 52 with the Cartesian G), and the final kernel multiplies by
+// the reciprocal vectors.  Bound by the latency of the table reads: the tables take
+// up to 64 KiB, so two blocks share a CU, of LF_THREADS threads each to have
+// waves enough.  256 atoms, 1.85 million G: 0.69 ms with the Cartesian G and 256
+// threads, 0.41 ms now.
 constexpr int LF_AG = 8;
+constexpr int LF_THREADS = 512;
 
 //   (+ conj(vxc_g) rhoc_s with a core density, :855-856)
 __global__ __launch_bounds__(256) void k_vtemp(int ngv, int nsp, const double* __restrict__ vps,
@@ -493,53 +504,64 @@ __global__ __launch_bounds__(256) void k_vtemp(int ngv, int nsp, const double* _
 }
 
 // grid (chunks, groups); partial[(a*nchunk + chunk)*3 + j]
-__global__ __launch_bounds__(256) void k_local_forces(
+__global__ __launch_bounds__(LF_THREADS) void k_local_forces(
     const int32_t* __restrict__ idx, int ngv, const double* __restrict__ tab, int krange,
     int kmin0, int kmin1, int kmin2, const int32_t* __restrict__ grp, const double* __restrict__ vt,
-    const double* __restrict__ gx, int chunk, double* __restrict__ partial) {
+    int chunk, double* __restrict__ partial) {
   extern __shared__ __align__(16) double ltab[];   // [LF_AG][3][krange][2]
   const int a0 = grp[3 * blockIdx.y], na = grp[3 * blockIdx.y + 1], is = grp[3 * blockIdx.y + 2];
   const int tsz = 3 * krange * 2;
-  for (int i = threadIdx.x; i < na * tsz; i += 256) ltab[i] = tab[(long)a0 * tsz + i];
+  for (int i = threadIdx.x; i < na * tsz; i += LF_THREADS) ltab[i] = tab[(long)a0 * tsz + i];
   __syncthreads();
   const int g0 = blockIdx.x * chunk, g1 = min(ngv, g0 + chunk);
   double v[3 * LF_AG];
 #pragma unroll
   for (int q = 0; q < 3 * LF_AG; q++) v[q] = 0.0;
   const double* vts = vt + 2 * (long)is * ngv;
-  for (int ig = g0 + threadIdx.x; ig < g1; ig += 256) {
+  for (int ig = g0 + threadIdx.x; ig < g1; ig += LF_THREADS) {
     const double vtr = vts[2 * ig], vti = vts[2 * ig + 1];
-    const double gxx = gx[ig], gyy = gx[ngv + ig], gzz = gx[2 * ngv + ig];
-    const int kx = idx[3 * ig] - kmin0, ky = idx[3 * ig + 1] - kmin1, kz = idx[3 * ig + 2] - kmin2;
+    const int k0 = idx[3 * ig], k1 = idx[3 * ig + 1], k2 = idx[3 * ig + 2];
+    const int kx = k0 - kmin0, ky = k1 - kmin1, kz = k2 - kmin2;
+    const double f0 = k0, f1 = k1, f2 = k2;
 #pragma unroll
     for (int q = 0; q < LF_AG; q++) {
       if (q < na) {
         double er, ei;
         eigr_from_tables(ltab + q * tsz, 0, krange, kx, ky, kz, er, ei);
         const double t = er * vti + ei * vtr;
-        v[3 * q] += t * gxx;
-        v[3 * q + 1] += t * gyy;
-        v[3 * q + 2] += t * gzz;
+        v[3 * q] += t * f0;
+        v[3 * q + 1] += t * f1;
+        v[3 * q + 2] += t * f2;
       }
     }
   }
   __shared__ double res[3 * LF_AG];
-  block_reduce_shfl<3 * LF_AG>(v, res);
+  block_reduce_shfl<3 * LF_AG, LF_THREADS / 64>(v, res);
   __syncthreads();
-  for (int i = threadIdx.x; i < 3 * na; i += 256)
+  for (int i = threadIdx.x; i < 3 * na; i += LF_THREADS)
     partial[((long)(a0 + i / 3) * gridDim.x + blockIdx.x) * 3 + i % 3] = res[i];
 }
 
-// sum chunks per atom: f[3a+j] = fion_esr[3a+j] - 2 omega sum_chunk partial
-__global__ void k_local_forces_final(const double* __restrict__ partial, int nchunk, int nat,
-                                     double omega, const double* __restrict__ fesr,
-                                     double* __restrict__ fion) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= 3 * nat) return;
-  const int a = t / 3, j = t % 3;
+// one block per atom: the chunks' sums (a wave each component: lanes take
+// the chunks, then a shuffle tree), times the reciprocal vectors b[3*axis + j]:
+// fion[3a+j] += fion_esr[3a+j] - 2 omega sum_axis b[axis][j] sum_axis
+__global__ __launch_bounds__(192) void k_local_forces_final(const double* __restrict__ partial,
+                                                            int nchunk, double omega,
+                                                            const double* __restrict__ b,
+                                                            const double* __restrict__ fesr,
+                                                            double* __restrict__ fion) {
+  __shared__ double sums[3];
+  const int a = blockIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double s = 0.0;
-  for (int c = 0; c < nchunk; c++) s += partial[((long)a * nchunk + c) * 3 + j];
-  fion[t] += fesr[t] + (-2.0 * omega) * s;
+  for (int c = lane; c < nchunk; c += 64) s += partial[((long)a * nchunk + c) * 3 + w];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  if (lane == 0) sums[w] = s;
+  __syncthreads();
+  const int j = threadIdx.x;
+  if (j < 3)
+    fion[3 * a + j] += fesr[3 * a + j] + (-2.0 * omega) * (b[j] * sums[0] + b[3 + j] * sums[1] +
+                                                           b[6 + j] * sums[2]);
 }
 
 // atoms per group: at most LF_AG, and their tables within 64 KiB of LDS
@@ -550,7 +572,7 @@ int local_forces_group_size(int krange) {
 void launch_local_forces(const int32_t* idx, int ngv, const double* tab, int krange,
                          const int* kmin, const int32_t* grp, int ngrp, int nsp,
                          const double* vps, const double* rhops, const double* g2i,
-                         const double* gx, const double* rhogt, const double* rhoelg,
+                         const double* b, const double* rhogt, const double* rhoelg,
                          const double* vxcg, const double* rhoc,
                          double omega, const double* fesr, int nat, double* vt, double* partial,
                          int nchunk, double* fion, hipStream_t s) {
@@ -558,10 +580,10 @@ void launch_local_forces(const int32_t* idx, int ngv, const double* tab, int kra
                      rhogt, rhoelg, vxcg, rhoc, vt);
   const int chunk = (ngv + nchunk - 1) / nchunk;
   const size_t lds = sizeof(double) * (size_t)local_forces_group_size(krange) * 3 * krange * 2;
-  hipLaunchKernelGGL(k_local_forces, dim3(nchunk, ngrp), dim3(256), lds, s, idx, ngv, tab,
-                     krange, kmin[0], kmin[1], kmin[2], grp, vt, gx, chunk, partial);
-  hipLaunchKernelGGL(k_local_forces_final, dim3((3 * nat + 255) / 256), dim3(256), 0, s,
-                     partial, nchunk, nat, omega, fesr, fion);
+  hipLaunchKernelGGL(k_local_forces, dim3(nchunk, ngrp), dim3(LF_THREADS), lds, s, idx, ngv, tab,
+                     krange, kmin[0], kmin[1], kmin[2], grp, vt, chunk, partial);
+  hipLaunchKernelGGL(k_local_forces_final, dim3(nat), dim3(192), 0, s, partial, nchunk, omega,
+                     b, fesr, fion);
 }
 
 // ------------------------------------------------------- projectors anl
@@ -742,14 +764,17 @@ __global__ __launch_bounds__(256) void k_nl_forces_y(
   block_reduce_store<3>(v, partial + ((long)a * gridDim.x + blockIdx.x) * 3);
 }
 
-__global__ void k_nl_forces_final(const double* __restrict__ partial, int nchunk, int nat,
-                                  double* __restrict__ fion) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
-  if (t >= 3 * nat) return;
-  const int a = t / 3, j = t % 3;
+// one block per atom, a wave each component: lanes take the chunks, then a
+// shuffle tree
+__global__ __launch_bounds__(192) void k_nl_forces_final(const double* __restrict__ partial,
+                                                         int nchunk,
+                                                         double* __restrict__ fion) {
+  const int a = blockIdx.x, j = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double s = 0.0;
-  for (int c = 0; c < nchunk; c++) s += partial[((long)a * nchunk + c) * 3 + j];
-  fion[t] -= 4.0 * s;
+  for (int c = lane; c < nchunk; c += 64) s += partial[((long)a * nchunk + c) * 3 + j];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
+  if (lane == 0) fion[3 * a + j] -= 4.0 * s;
 }
 
 // the fused force product's partials: sum over the row tiles in a fixed-order
@@ -788,8 +813,7 @@ void launch_nl_forces_y(const T* A, const T* Y, long lda, int ngw, const double*
   const int chunk = (ngw + nchunk - 1) / nchunk;
   hipLaunchKernelGGL(k_nl_forces_y<T>, dim3(nchunk, nat), dim3(256), 0, s, A, Y, lda, ngw, gx, a_m0,
                      a_npr, a_stride, chunk, partial);
-  hipLaunchKernelGGL(k_nl_forces_final, dim3((3 * nat + 255) / 256), dim3(256), 0, s, partial,
-                     nchunk, nat, fion);
+  hipLaunchKernelGGL(k_nl_forces_final, dim3(nat), dim3(192), 0, s, partial, nchunk, fion);
 }
 template void launch_nl_forces_y<double>(const double*, const double*, long, int, const double*,
                                          const int32_t*, const int32_t*, const int32_t*, int,
@@ -870,14 +894,24 @@ __global__ __launch_bounds__(256) void k_nl_stress_y(
   block_reduce_store<6>(v, partial + ((long)s * gridDim.x + blockIdx.x) * 6);
 }
 
-// out6[ij] = 4 * sum of the partials (fixed order)
-__global__ void k_nl_stress_final(const double* __restrict__ partial, int nblk,
-                                  double* __restrict__ out6) {
-  const int ij = threadIdx.x;
-  if (ij >= 6) return;
-  double s = 0.0;
-  for (int b = 0; b < nblk; b++) s += partial[(long)b * 6 + ij];
-  out6[ij] = 4.0 * s;
+// out6[ij] = 4 * sum of the partials: one block per component, a strided
+// slice per thread, then a tree
+__global__ __launch_bounds__(256) void k_nl_stress_final(const double* __restrict__ partial,
+                                                         int nblk, double* __restrict__ out6) {
+  const int ij = blockIdx.x;
+  double v[1] = {0.0};
+  for (int b = threadIdx.x; b < nblk; b += 256) v[0] += partial[(long)b * 6 + ij];
+  __shared__ double res[1];
+  block_reduce_store<1>(v, res);
+  __syncthreads();
+  if (threadIdx.x == 0) out6[ij] = 4.0 * res[0];
+}
+
+// chunks of G per species: one vector per thread (the atoms of a species
+// are a loop of sincos in each thread, so 64 chunks left most CUs idle: 128 atoms,
+// 105502 G: 1.51 ms, 0.31 with these), at most NLS_CHUNKS_MAX
+int nl_stress_chunks(int ngw) {
+  return std::max(1, std::min(NLS_CHUNKS_MAX, (ngw + 255) / 256));
 }
 
 template <typename T>
@@ -885,22 +919,23 @@ void launch_nl_stress_y(const T* Y, long lda, int ngw, const double* gx, const d
                         int nsp, const int32_t* sp_first, const int32_t* sp_npr,
                         const int64_t* dt_off, const double* dtwnl, const int32_t* a_m0,
                         const int32_t* a_stride, const int32_t* m_l, double* partial,
-                        int nchunk, double* out6, hipStream_t s, int halves, long mhalf) {
+                        double* out6, hipStream_t s, int halves, long mhalf) {
+  const int nchunk = nl_stress_chunks(ngw);
   const int chunk = (ngw + nchunk - 1) / nchunk;
   hipLaunchKernelGGL(k_nl_stress_y<T>, dim3(nchunk, nsp), dim3(256), 0, s, Y, lda, ngw, gx, tau,
                      sp_first, sp_npr, dt_off, dtwnl, a_m0, a_stride, m_l, chunk, halves, mhalf,
                      partial);
-  hipLaunchKernelGGL(k_nl_stress_final, dim3(1), dim3(64), 0, s, partial, nchunk * nsp, out6);
+  hipLaunchKernelGGL(k_nl_stress_final, dim3(6), dim3(256), 0, s, partial, nchunk * nsp, out6);
 }
 template void launch_nl_stress_y<double>(const double*, long, int, const double*, const double*,
                                          int, const int32_t*, const int32_t*, const int64_t*,
                                          const double*, const int32_t*, const int32_t*,
-                                         const int32_t*, double*, int, double*, hipStream_t,
+                                         const int32_t*, double*, double*, hipStream_t,
                                          int, long);
 template void launch_nl_stress_y<float>(const float*, long, int, const double*, const double*,
                                         int, const int32_t*, const int32_t*, const int64_t*,
                                         const double*, const int32_t*, const int32_t*,
-                                        const int32_t*, double*, int, double*, hipStream_t,
+                                        const int32_t*, double*, double*, hipStream_t,
                                         int, long);
 
 // ------------------------------------------- Hartree pseudocharge stress
