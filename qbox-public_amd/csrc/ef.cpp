@@ -1935,26 +1935,26 @@ int qbg_gram(qbg_ctx* c, double* cc, int ldc, int ngw, int nst, int prec) {
     const long K = 2L * ngw;
     const int tm = (nst + 63) / 64;
     const size_t work = (size_t)nst * nst * std::max(1, 2048 / (tm * tm) + 1);
-    double *S = nullptr, *X = nullptr, *T = nullptr, *W = nullptr;
+    const long ldx = 2L * nst;           // S on top of X (chol_inverse)
+    double *S = nullptr, *T = nullptr, *W = nullptr;
     int* info = nullptr;
     int rc = QBG_OK;
-    if ((rc = dalloc(c, &S, (size_t)nst * nst)) || (rc = dalloc(c, &X, (size_t)nst * nst)) ||
-        (rc = dalloc(c, &T, (size_t)K * nst)) || (rc = dalloc(c, &W, work)) ||
-        (rc = dalloc(c, &info, 1))) {
-      (void)hipFree(S); (void)hipFree(X); (void)hipFree(T); (void)hipFree(W); (void)hipFree(info);
+    if ((rc = dalloc(c, &S, (size_t)ldx * nst)) || (rc = dalloc(c, &T, (size_t)K * nst)) ||
+        (rc = dalloc(c, &W, work)) || (rc = dalloc(c, &info, 1))) {
+      (void)hipFree(S); (void)hipFree(T); (void)hipFree(W); (void)hipFree(info);
       return rc;
     }
     auto release = [&]() {
-      (void)hipFree(S); (void)hipFree(X); (void)hipFree(T); (void)hipFree(W); (void)hipFree(info);
+      (void)hipFree(S); (void)hipFree(T); (void)hipFree(W); (void)hipFree(info);
     };
     c->prof_begin(QBG_K_GRAM);
     cleanup(cc, ldc, nst, s);
-    if (gemm_syrk(cc, 2L * ldc, nst, K, 2.0, -1.0, S, nst, W, work, s)) {
+    if (gemm_syrk(cc, 2L * ldc, nst, K, 2.0, -1.0, S, ldx, W, work, s)) {
       (void)hipStreamSynchronize(s);
       release();
       return c->fail(QBG_E_INVAL, "gram workspace");
     }
-    potrf(S, nst, nst, info, s, W);
+    chol_inverse(S, nst, nullptr, info, W, s);
     c->prof_end();
     // the coefficients are only touched once the factorization succeeded
     // (the reference aborts in potrf, src/Matrix.cpp:2324-2327)
@@ -1967,8 +1967,7 @@ int qbg_gram(qbg_ctx* c, double* cc, int ldc, int ngw, int nst, int prec) {
       return c->fail(QBG_E_NOT_SPD, "gram: overlap matrix not positive definite");
     }
     c->prof_begin(QBG_K_GRAM);
-    trtri(S, nst, nst, X, s);
-    gemm_nn_triu(cc, 2L * ldc, X, nst, K, nst, T, K, s);
+    gemm_nn_triu(cc, 2L * ldc, S + nst, ldx, K, nst, T, K, s);
     (void)hipMemcpy2DAsync(cc, sizeof(double) * 2 * ldc, T, sizeof(double) * K, sizeof(double) * K,
                            nst, hipMemcpyDeviceToDevice, s);
     c->prof_end();

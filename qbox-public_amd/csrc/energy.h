@@ -101,16 +101,25 @@ int gemm_tn_splitk(const double* A, long lda, const double* B, long ldb, int M, 
 int gemm_tn_splitk(const float* A, long lda, const double* B, long ldb, int M, int N, long K,
                    double alpha, double gamma, double* out, long ldo, double* work,
                    size_t work_doubles, int prec, hipStream_t s);
+// what the sum over the splits of a product adds to the output: delta I + beta
+// (the output before), and, if T, a second output T = I + 3/4 out with the same
+// leading dimension and split_blocks(M N) partial sums of the squares of out
+struct SplitEnd {
+  double delta = 0.0, beta = 0.0;
+  double *T = nullptr, *part = nullptr;
+};
+int split_blocks(long outputs);
 // symmetric TN (FP64): out = alpha A^T A + gamma a0 a0^T, only the lower
 // tiles formed, the upper part mirrored
 int gemm_syrk(const double* A, long lda, int N, long K, double alpha, double gamma, double* out,
               long ldo, double* work, size_t work_doubles, hipStream_t s,
-              const int* skip = nullptr);
+              const int* skip = nullptr, const SplitEnd& end = {});
 // NN (FP64) split over the reduction for small outputs (partials in work):
-// C[k + n*ldc] = sum_m A[k + m*lda] F[m + n*ldf].  Returns -1 on a bad shape.
+// C[k + n*ldc] = alpha sum_m A[k + m*lda] F[m + n*ldf].  C may be A or F: the sum
+// over the splits writes it.  Returns -1 on a bad shape.
 int gemm_nn_splitk(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
                    double* C, long ldc, double* work, size_t work_doubles, hipStream_t s,
-                   const int* skip = nullptr);
+                   const int* skip = nullptr, double alpha = 1.0, const SplitEnd& end = {});
 // NN (FP64) whose output columns may be columns of A, N <= gemm_nn_tile_p():
 // one block holds all N columns of its rows and reads them before it writes
 int gemm_nn_tile_p();
@@ -168,15 +177,14 @@ void convert_f32(const double* c, long ldc2, long K, int nst, float* c32, long l
 void fout_f32(const double* fout, const double* occ, int M, int nst, float* f32, long ldf,
               float* w32, long ldw, hipStream_t s, int nzero = 0);
 
-// lower Cholesky in place; info[0] = 0 or the failing pivot + 1.  With a
-// workspace of 64 * n doubles (ws) the factorization runs blocked over the
-// whole device, otherwise in one work-group
-void potrf(double* S, int n, int lds, int* info, hipStream_t s, double* ws = nullptr);
-// the blocked factorization for any n (ws: 64 * n doubles); info = -1 and
-// nothing done when *skip
-void potrf_device(double* S, int n, int lds, int* info, double* ws, hipStream_t s,
-                  const int* skip);
-void trtri(const double* L, int n, int ldl, double* X, hipStream_t s, const int* skip = nullptr);
+// SX: 2n x n, column-major, leading dimension 2n.  Its rows 0 .. n-1 hold a symmetric S,
+// or S = I - q is formed there (q, n x n); they are overwritten.  Its rows
+// n .. 2n-1 become X = L^-T (upper triangular, zero below), S = L L^T.
+// info[0] = 0, or the failing pivot + 1 (X is then not usable), or -1 and
+// nothing else done when *skip.  ws: CHOL_PANEL n doubles if n > CHOL_PANEL.
+constexpr int CHOL_PANEL = 64;
+void chol_inverse(double* SX, int n, const double* q, int* info, double* ws, hipStream_t s,
+                  const int* skip = nullptr);
 void cleanup(double* c, long ldc, int nst, hipStream_t s);
 
 }  // namespace qbg

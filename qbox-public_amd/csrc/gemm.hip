@@ -1,7 +1,6 @@
-// gemm.hip -- MFMA GEMMs and the small dense factorizations of the
-// projector path (NonLocalPotential::energy dgemm calls,
-// src/NonLocalPotential.cpp:1411-1428, 1611, 1716) and of SlaterDet::gram
-// (syrk/syr/potrf/trsm, src/SlaterDet.cpp:487-520).
+// gemm.hip -- MFMA GEMMs of the projector path (NonLocalPotential::energy
+// dgemm calls, src/NonLocalPotential.cpp:1411-1428, 1611, 1716) and of
+// SlaterDet::gram (syrk/syr, src/SlaterDet.cpp:487-520).
 //
 // One kernel shape serves every product: D[p][q] = sum_r P(r,p) Q(r,q) on a
 // (32 BI) x (32 BJ) tile per block of 256 threads: 2x2 waves, each a BI x BJ
@@ -261,8 +260,9 @@ __global__ __launch_bounds__(256, 2) void k_gemm(GemmArgs g) {
       }
 }
 
-// out[q + p*ldo] = alpha * sum_s partial[s][p][q] + gamma * Q[q*ldq] * P[p*ldp].
-// A block sums 64 outputs: wave y takes the splits y, y + 4, ... (eight loads
+// out[q + p*ldo] = alpha * sum_s partial[s][p][q] + gamma * Q[q*ldq] * P[p*ldp]
+// + delta (p = q) + beta * out; if T: T (as out) = I + 3/4 out, and the sum of
+// the squares of a block's outputs to part.  A block sums 64 outputs: wave y takes the splits y, y + 4, ... (eight loads
 // in flight), and the four sums are added in that order.
 template <typename TQm, typename TPm>
 __global__ __launch_bounds__(256) void k_split_reduce(const double* __restrict__ partial, int S,
@@ -270,7 +270,8 @@ __global__ __launch_bounds__(256) void k_split_reduce(const double* __restrict__
                                                       const TQm* __restrict__ Q, long ldq,
                                                       const TPm* __restrict__ P, long ldp,
                                                       double* __restrict__ out, long ldo,
-                                                      int sym, const int* __restrict__ skip) {
+                                                      int sym, const int* __restrict__ skip,
+                                                      SplitEnd end) {
   if (skip && *skip) return;
   __shared__ double sums[4][64];
   const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
@@ -285,10 +286,23 @@ __global__ __launch_bounds__(256) void k_split_reduce(const double* __restrict__
   }
   sums[y][x] = s;
   __syncthreads();
-  if (y || t >= tot) return;
-  double v = alpha * ((sums[0][x] + sums[1][x]) + (sums[2][x] + sums[3][x]));
-  if (gamma != 0.0) v += gamma * (double)Q[(long)q * ldq] * (double)P[(long)p * ldp];
-  out[q + (long)p * ldo] = v;
+  if (y) return;
+  double v = 0.0;
+  if (t < tot) {
+    v = alpha * ((sums[0][x] + sums[1][x]) + (sums[2][x] + sums[3][x]));
+    if (gamma != 0.0) v += gamma * (double)Q[(long)q * ldq] * (double)P[(long)p * ldp];
+    if (p == q) v += end.delta;
+    double* o = out + q + (long)p * ldo;
+    if (end.beta != 0.0) v += end.beta * *o;
+    *o = v;
+    if (end.T) end.T[q + (long)p * ldo] = (p == q ? 1.0 : 0.0) + 0.75 * v;
+  }
+  if (end.T) {
+    double r = v * v;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) r += __shfl_down(r, off, 64);
+    if (x == 0) end.part[blockIdx.x] = r;
+  }
 }
 
 namespace {
@@ -384,7 +398,8 @@ constexpr unsigned BJ_TN = 0x1e, BJ_NN = 0x16;   // compiled bj of the two forms
 template <typename TQm>
 int tn_splitk(const TQm* A, long lda, const double* B, long ldb, int M, int N, long K,
               double alpha, double gamma, double* out, long ldo, double* work,
-              size_t work_doubles, int prec, int sym, hipStream_t s, const int* skip) {
+              size_t work_doubles, int prec, int sym, hipStream_t s, const int* skip,
+              const SplitEnd& end = {}) {
   if (M <= 0 || N <= 0 || K <= 0) return -1;
   if ((size_t)M * N > work_doubles || (sizeof(TQm) == 4 && prec == QBG_PREC_FP64)) return -1;
   GemmArgs g{};
@@ -406,7 +421,7 @@ int tn_splitk(const TQm* A, long lda, const double* B, long ldb, int M, int N, l
   const long tot = (long)M * N;
   hipLaunchKernelGGL((k_split_reduce<TQm, double>), dim3((unsigned)((tot + 63) / 64)),
                      dim3(256), 0, s, work, (int)S, M, N, alpha, gamma, A, lda, B, ldb, out, ldo,
-                     sym, skip);
+                     sym, skip, end);
   return 0;
 }
 
@@ -438,7 +453,7 @@ void nn(const TQm* A, long lda, const double* F, long ldf, long K, int N, int M,
 // C[k + n*ldc] = sum_m A[k + m*lda] F[m + n*ldf]
 int gemm_nn_splitk(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
                    double* C, long ldc, double* work, size_t work_doubles, hipStream_t s,
-                   const int* skip) {
+                   const int* skip, double alpha, const SplitEnd& end) {
   if (K <= 0 || N <= 0 || M <= 0) return -1;
   if ((size_t)K * N > work_doubles) return -1;
   GemmArgs g{};
@@ -456,8 +471,8 @@ int gemm_nn_splitk(const double* A, long lda, const double* F, long ldf, long K,
   launch_gemm<double, double, double, false, double>(g, k, s);
   const long tot = K * N;
   hipLaunchKernelGGL((k_split_reduce<double, double>), dim3((unsigned)((tot + 63) / 64)),
-                     dim3(256), 0, s, work, (int)S, (int)K, N, 1.0, 0.0, A, lda, F, ldf, C, ldc,
-                     0, skip);
+                     dim3(256), 0, s, work, (int)S, (int)K, N, alpha, 0.0, A, lda, F, ldf, C, ldc,
+                     0, skip, end);
   return 0;
 }
 int gemm_tn_splitk(const double* A, long lda, const double* B, long ldb, int M, int N, long K,
@@ -473,10 +488,12 @@ int gemm_tn_splitk(const float* A, long lda, const double* B, long ldb, int M, i
                    s, nullptr);
 }
 int gemm_syrk(const double* A, long lda, int N, long K, double alpha, double gamma, double* out,
-              long ldo, double* work, size_t work_doubles, hipStream_t s, const int* skip) {
+              long ldo, double* work, size_t work_doubles, hipStream_t s, const int* skip,
+              const SplitEnd& end) {
   return tn_splitk(A, lda, A, lda, N, N, K, alpha, gamma, out, ldo, work, work_doubles,
-                   QBG_PREC_FP64, 1, s, skip);
+                   QBG_PREC_FP64, 1, s, skip, end);
 }
+int split_blocks(long outputs) { return (int)((outputs + 63) / 64); }
 int gemm_nn_tile_p() { return 128; }
 void gemm_nn_triu(const double* A, long lda, const double* F, long ldf, long K, int N, double* C,
                   long ldc, hipStream_t s) {
@@ -497,282 +514,6 @@ void gemm_nn(const float* A, long lda, const double* F, long ldf, long K, int N,
 void gemm_nn(const double* A, long lda, const double* F, long ldf, long K, int N, int M,
              float* C, long ldc, int accumulate, int prec, hipStream_t s) {
   nn(A, lda, F, ldf, K, N, M, C, ldc, accumulate, prec, 0, 0, s, nullptr);
-}
-
-// ------------------------------------------------------- Cholesky, inverse
-// In-place lower Cholesky of the column-major n x n matrix S (right-looking,
-// one work-group).  info[0] = 0, or j+1 if pivot j is not positive
-// (src/Matrix.cpp:2308-2334 returns info from dpotrf the same way).
-__global__ __launch_bounds__(1024) void k_potrf(double* __restrict__ S, int n, int lds,
-                                                int* __restrict__ info) {
-  __shared__ double piv;
-  __shared__ int bad;
-  if (threadIdx.x == 0) bad = 0;
-  __syncthreads();
-  for (int j = 0; j < n; j++) {
-    if (threadIdx.x == 0) {
-      const double d = S[j + (long)j * lds];
-      if (!(d > 0.0)) { bad = j + 1; piv = 1.0; }
-      else piv = sqrt(d);
-      S[j + (long)j * lds] = piv;
-    }
-    __syncthreads();
-    if (bad) break;
-    const double p = piv;
-    for (int i = j + 1 + threadIdx.x; i < n; i += blockDim.x) S[i + (long)j * lds] /= p;
-    __syncthreads();
-    // trailing update of the lower triangle: S[i][c] -= L[i][j] L[c][j], c<=i
-    const int m = n - j - 1;
-    const long tot = (long)m * (m + 1) / 2;
-    for (long t = threadIdx.x; t < tot; t += blockDim.x) {
-      // t -> (i, c) with c <= i in the trailing block, row-wise packing
-      int i = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
-      while ((long)i * (i + 1) / 2 > t) i--;
-      while ((long)(i + 1) * (i + 2) / 2 <= t) i++;
-      const int cc = (int)(t - (long)i * (i + 1) / 2);
-      const int gi = j + 1 + i, gc = j + 1 + cc;
-      S[gi + (long)gc * lds] -= S[gi + (long)j * lds] * S[gc + (long)j * lds];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) info[0] = bad;
-}
-
-// Blocked lower Cholesky in one work-group: panels of PB columns.  Per
-// panel the PB x PB diagonal block is factored in LDS, the rows below are
-// solved against it (one thread per row) and kept in LDS, and the trailing
-// lower triangle is updated from LDS.  info as for k_potrf.
-constexpr int PB = 8;
-constexpr int POTRF_NMAX = 960;    // rows of the LDS panel
-
-__global__ __launch_bounds__(1024) void k_potrf_blk(double* __restrict__ S, int n, int lds,
-                                                    int* __restrict__ info) {
-  __shared__ double D[PB][PB + 1];
-  __shared__ double P[POTRF_NMAX * PB];
-  __shared__ int bad;
-  const int tid = threadIdx.x;
-  if (tid == 0) bad = 0;
-  __syncthreads();
-  for (int j0 = 0; j0 < n; j0 += PB) {
-    const int nb = min(PB, n - j0), j1 = j0 + nb, rows = n - j1;
-    if (tid < nb * nb) D[tid / nb][tid % nb] = S[(j0 + tid / nb) + (long)(j0 + tid % nb) * lds];
-    __syncthreads();
-    if (tid == 0) {                        // unblocked factor of the diagonal block
-      for (int c = 0; c < nb && !bad; c++) {
-        double d = D[c][c];
-        for (int t = 0; t < c; t++) d -= D[c][t] * D[c][t];
-        if (!(d > 0.0)) { bad = j0 + c + 1; break; }
-        d = sqrt(d);
-        D[c][c] = d;
-        for (int r = c + 1; r < nb; r++) {
-          double v = D[r][c];
-          for (int t = 0; t < c; t++) v -= D[r][t] * D[c][t];
-          D[r][c] = v / d;
-        }
-      }
-    }
-    __syncthreads();
-    if (bad) break;
-    if (tid < nb * nb && tid / nb >= tid % nb)
-      S[(j0 + tid / nb) + (long)(j0 + tid % nb) * lds] = D[tid / nb][tid % nb];
-    // rows below: L_i = A_i D^-T (forward substitution)
-    for (int i = tid; i < rows; i += blockDim.x) {
-      double x[PB];
-#pragma unroll
-      for (int c = 0; c < PB; c++) {
-        if (c < nb) {
-          double v = S[(j1 + i) + (long)(j0 + c) * lds];
-          for (int t = 0; t < c; t++) v -= x[t] * D[c][t];
-          x[c] = v / D[c][c];
-          S[(j1 + i) + (long)(j0 + c) * lds] = x[c];
-          P[i * PB + c] = x[c];
-        }
-      }
-    }
-    __syncthreads();
-    // trailing lower triangle: A_ik -= L_i . L_k, k <= i
-    for (long t = tid; t < (long)rows * rows; t += blockDim.x) {
-      const int i = (int)(t / rows), k = (int)(t - (long)i * rows);
-      if (k <= i) {
-        double v = 0.0;
-        for (int c = 0; c < nb; c++) v += P[i * PB + c] * P[k * PB + c];
-        S[(j1 + i) + (long)(j1 + k) * lds] -= v;
-      }
-    }
-    __syncthreads();
-  }
-  if (tid == 0) info[0] = bad;
-}
-
-// Right-looking blocked Cholesky over the whole device, panels of CB
-// columns: the diagonal block factored in LDS by one work-group, the rows
-// below solved against it (one row per thread), and the trailing matrix
-// updated by an MFMA GEMM with the panel's negated transpose kept in ws.
-// info as for k_potrf; after a failure the remaining launches do nothing.
-constexpr int CB = 64;
-
-// info = 0, or -1 when *skip (every later launch of the factorization then
-// does nothing)
-__global__ void k_init_info(int* p, const int* skip) {
-  if (threadIdx.x == 0) *p = (skip && *skip) ? -1 : 0;
-}
-
-__global__ __launch_bounds__(256) void k_chol_diag(double* __restrict__ S, int lds, int j0,
-                                                   int jb, int* __restrict__ info) {
-  if (*info) return;
-  __shared__ double D[CB][CB + 1];
-  __shared__ int bad;
-  const int tid = threadIdx.x;
-  for (int e = tid; e < jb * jb; e += 256) D[e % jb][e / jb] = S[(j0 + e % jb) + (long)(j0 + e / jb) * lds];
-  if (tid == 0) bad = 0;
-  __syncthreads();
-  for (int c = 0; c < jb; c++) {
-    const double d = D[c][c];
-    if (!(d > 0.0)) {                      // uniform: every thread read D[c][c]
-      if (tid == 0) *info = j0 + c + 1;
-      return;
-    }
-    const double sd = sqrt(d);
-    __syncthreads();
-    if (tid == 0) D[c][c] = sd;
-    for (int r = c + 1 + tid; r < jb; r += 256) D[r][c] /= sd;
-    __syncthreads();
-    // D[r][k] -= D[r][c] D[k][c], c < k <= r
-    const int m = jb - c - 1;
-    for (int e = tid; e < m * m; e += 256) {
-      const int r = c + 1 + e / m, k = c + 1 + e % m;
-      if (k <= r) D[r][k] -= D[r][c] * D[k][c];
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < jb * jb; e += 256) {
-    const int r = e % jb, k = e / jb;
-    if (k <= r) S[(j0 + r) + (long)(j0 + k) * lds] = D[r][k];
-  }
-}
-
-__global__ __launch_bounds__(64) void k_chol_panel(double* __restrict__ S, int n, int lds, int j0,
-                                                   int jb, const int* __restrict__ info,
-                                                   double* __restrict__ lt) {
-  if (*info) return;
-  __shared__ double D[CB][CB + 1];
-  const int tid = threadIdx.x;
-  for (int e = tid; e < jb * jb; e += 64) D[e % jb][e / jb] = S[(j0 + e % jb) + (long)(j0 + e / jb) * lds];
-  __syncthreads();
-  const int j1 = j0 + jb, i = blockIdx.x * 64 + tid;
-  if (j1 + i >= n) return;
-  double x[CB];
-#pragma unroll
-  for (int c = 0; c < CB; c++) {
-    if (c < jb) {
-      double v = S[(j1 + i) + (long)(j0 + c) * lds];
-#pragma unroll
-      for (int t = 0; t < c; t++) v -= x[t] * D[c][t];
-      x[c] = v / D[c][c];
-      S[(j1 + i) + (long)(j0 + c) * lds] = x[c];
-      lt[c + (long)i * CB] = -x[c];
-    }
-  }
-}
-
-static void potrf_blocked(double* S, int n, int lds, int* info, double* ws, hipStream_t s,
-                          const int* skip) {
-  hipLaunchKernelGGL(k_init_info, dim3(1), dim3(64), 0, s, info, skip);
-  for (int j0 = 0; j0 < n; j0 += CB) {
-    const int jb = std::min(CB, n - j0), rows = n - j0 - jb;
-    hipLaunchKernelGGL(k_chol_diag, dim3(1), dim3(256), 0, s, S, lds, j0, jb, info);
-    if (rows <= 0) break;
-    hipLaunchKernelGGL(k_chol_panel, dim3((rows + 63) / 64), dim3(64), 0, s, S, n, lds, j0, jb,
-                       info, ws);
-    // A22 += L21 (-L21^T)
-    nn(S + (j0 + jb) + (long)j0 * lds, lds, ws, CB, rows, rows, jb, S + (j0 + jb) +
-       (long)(j0 + jb) * lds, lds, 1, QBG_PREC_FP64, 0, 0, s, info);
-  }
-}
-
-void potrf_device(double* S, int n, int lds, int* info, double* ws, hipStream_t s,
-                  const int* skip) {
-  potrf_blocked(S, n, lds, info, ws, s, skip);
-}
-
-// X = L^{-1} (lower), written row-major (X[i*n + c], upper part zero):
-// block column J of TB columns per work-group, X_IJ = L_II^{-1} (E_IJ -
-// sum_{J <= K < I} L_IK X_KJ) for I = J, J+1, ... with 32 x 32 tiles staged
-// in LDS; one wave solves the diagonal-block system column by column.
-constexpr int TB = 32;
-__global__ __launch_bounds__(256) void k_trtri_blk(const double* __restrict__ L, int n, int ldl,
-                                                   double* __restrict__ X,
-                                                   const int* __restrict__ skip) {
-  if (skip && *skip) return;
-  __shared__ double R[TB][TB + 1];
-  __shared__ double La[TB][TB + 1];
-  __shared__ double Xb[TB][TB + 1];
-  const int tid = threadIdx.x, J = blockIdx.x, nbk = (n + TB - 1) / TB;
-  const int c0 = J * TB;
-  // upper blocks of this block column are zero
-  for (long t = tid; t < (long)c0 * TB; t += 256) {
-    const int r = (int)(t / TB), c = c0 + (int)(t % TB);
-    if (c < n) X[(long)r * n + c] = 0.0;
-  }
-  for (int I = J; I < nbk; I++) {
-    const int r0 = I * TB;
-    for (int e = tid; e < TB * TB; e += 256) {
-      const int r = e / TB, c = e % TB;
-      R[r][c] = (I == J && r == c) ? 1.0 : 0.0;
-    }
-    for (int K = J; K < I; K++) {
-      const int k0 = K * TB;
-      __syncthreads();
-      for (int e = tid; e < TB * TB; e += 256) {
-        const int r = e / TB, c = e % TB;
-        La[r][c] = (r0 + r < n && k0 + c < n) ? L[(r0 + r) + (long)(k0 + c) * ldl] : 0.0;
-        Xb[r][c] = (k0 + r < n && c0 + c < n) ? X[(long)(k0 + r) * n + c0 + c] : 0.0;
-      }
-      __syncthreads();
-      for (int e = tid; e < TB * TB; e += 256) {
-        const int r = e / TB, c = e % TB;
-        double v = 0.0;
-#pragma unroll 8
-        for (int t = 0; t < TB; t++) v += La[r][t] * Xb[t][c];
-        R[r][c] -= v;
-      }
-    }
-    __syncthreads();
-    for (int e = tid; e < TB * TB; e += 256) {
-      const int r = e / TB, c = e % TB;
-      La[r][c] = (r0 + r < n && r0 + c < n) ? L[(r0 + r) + (long)(r0 + c) * ldl]
-                                            : (r == c ? 1.0 : 0.0);
-    }
-    __syncthreads();
-    if (tid < TB) {                       // column tid: forward substitution
-      const int c = tid;
-      for (int r = 0; r < TB; r++) {
-        double v = R[r][c];
-        for (int t = 0; t < r; t++) v -= La[r][t] * R[t][c];
-        R[r][c] = v / La[r][r];
-      }
-    }
-    __syncthreads();
-    for (int e = tid; e < TB * TB; e += 256) {
-      const int r = e / TB, c = e % TB;
-      if (r0 + r < n && c0 + c < n) X[(long)(r0 + r) * n + c0 + c] = R[r][c];
-    }
-    __syncthreads();                      // X of this step is read in the next
-  }
-}
-
-void potrf(double* S, int n, int lds, int* info, hipStream_t s, double* ws) {
-  if (ws && n > 2 * CB) {
-    potrf_blocked(S, n, lds, info, ws, s, nullptr);
-    return;
-  }
-  if (n <= POTRF_NMAX)
-    hipLaunchKernelGGL(k_potrf_blk, dim3(1), dim3(1024), 0, s, S, n, lds, info);
-  else
-    hipLaunchKernelGGL(k_potrf, dim3(1), dim3(1024), 0, s, S, n, lds, info);
-}
-void trtri(const double* L, int n, int ldl, double* X, hipStream_t s, const int* skip) {
-  hipLaunchKernelGGL(k_trtri_blk, dim3((n + TB - 1) / TB), dim3(256), 0, s, L, n, ldl, X, skip);
 }
 
 // zero Im c(G=0) of every band (SlaterDet::cleanup, src/SlaterDet.cpp:1335-1356)

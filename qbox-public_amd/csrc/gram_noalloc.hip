@@ -75,29 +75,29 @@ int qbg_gram_noalloc(qbg_ctx* c, double* cc, int ldc, int ngw, int nst, int prec
     hipStream_t s = c->stream;
     const long K = 2L * ngw, lda = 2L * ldc;
     const size_t nn = (size_t)nst * nst;
-    double* S = base;
-    double* X = S + nn;
-    double* W = X + nn;
+    const long ldx = 2L * nst;
+    double* S = base;                  // rows 0 .. nst-1 of a 2 nst x nst array, X below
+    double* X = S + nst;
+    double* W = S + 2 * nn;
     const size_t work = (size_t)QBG_GRAM_NOALLOC_SPLITS * nn;
     int* info = reinterpret_cast<int*>(W + work);
     c->prof_begin(QBG_K_GRAM);
     qbg::cleanup(cc, ldc, nst, s);
-    if (qbg::gemm_syrk(cc, lda, nst, K, 2.0, -1.0, S, nst, W, work, s))
+    if (qbg::gemm_syrk(cc, lda, nst, K, 2.0, -1.0, S, ldx, W, work, s))
       return c->fail(QBG_E_INVAL, "gram_noalloc: overlap workspace");
-    qbg::potrf(S, nst, nst, info, s, W);
+    qbg::chol_inverse(S, nst, nullptr, info, W, s);
     c->prof_end();
     int hinfo = 0;
     QBG_HIP(c, hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, s));
     QBG_HIP(c, hipStreamSynchronize(s));
     if (hinfo) return c->fail(QBG_E_NOT_SPD, "gram: overlap matrix not positive definite");
     c->prof_begin(QBG_K_GRAM);
-    qbg::trtri(S, nst, nst, X, s);
-    // X = L^-1 row-major is L^-T column-major (upper triangular):
+    // X = L^-T (upper triangular):
     // C[:, j0:j1] = C[:, 0:j1] X[0:j1, j0:j1], last block first
     const int tp = qbg::gemm_nn_tile_p();
     for (int j0 = ((nst - 1) / tp) * tp; j0 >= 0; j0 -= tp) {
       const int j1 = std::min(nst, j0 + tp);
-      qbg::gemm_nn_inplace(cc, lda, X + (size_t)j0 * nst, nst, K, j1 - j0, j1,
+      qbg::gemm_nn_inplace(cc, lda, X + (size_t)j0 * ldx, ldx, K, j1 - j0, j1,
                            cc + (size_t)j0 * lda, lda, s);
     }
     c->prof_end();

@@ -44,21 +44,27 @@ void launch_copy_cols_if(double* dst, long lddst, const double* src, long ldsrc,
 // flags: [0] done, [1] skip Bjorck-Bowie step, [2] skip Higham step,
 //        [3] iterations, [4] singular, [5] Cholesky status of a Higham step
 void launch_polar_init(int* flags, hipStream_t s);
-// q = q_in + I (q_in = -x^T x), its Frobenius norm; sets flags for this step
-void launch_polar_norm(double* q, int n, double tol, int* flags, double* qnrm, hipStream_t s);
-// t = I + a q (elementwise on the n x n matrix), skipped when *skip
-void launch_ident_axpy(double* t, const double* q, int n, double a, const int* skip,
+// ||q||_F from npart partial sums of the squares of q = I - x^T x; sets flags for this step
+void launch_polar_norm(const double* part, int npart, double tol, int* flags, double* qnrm,
                        hipStream_t s);
-// dst = src (n x n), skipped when *skip
-void launch_copy_if_not(double* dst, const double* src, long count, const int* skip,
-                        hipStream_t s);
 // Higham step helpers (x^-T = x (x^T x)^-1 through the blocked Cholesky):
-// dst = transpose of src (n x n), x = (x + z) / 2, flags[4] = 1 if *info > 0;
-// the first two skipped when *skip
+// dst = transpose of src (n x n, src's columns lds apart), skipped when *skip;
+// flags[4] = 1 if *info > 0
 constexpr int POLAR_NMAX = 4096;
-void launch_transpose_if(double* dst, const double* src, int n, const int* skip, hipStream_t s);
-void launch_higham_update(double* x, const double* z, int n, const int* skip, hipStream_t s);
+void launch_transpose_if(double* dst, const double* src, int n, long lds, const int* skip,
+                         hipStream_t s);
 void launch_polar_singular(const int* info, int* flags, hipStream_t s);
+
+// the whole iteration as one launch of one work-group, for n <= POLAR_ONE:
+// there the launches of the general sequence, 14 and more for each of maxiter steps
+// whether taken or skipped, cost more than one CU's product rate (three steps
+// 0.27 ms at n = 128, 1.25 ms at n = 129; five with Higham's 0.58 and 1.24), and one matrix
+// fits in LDS.
+// y1, y2, lt: polar_elems(n) doubles each, sx: twice that
+constexpr int POLAR_ONE = 128;
+size_t polar_elems(int n);      // of one buffer of the iteration, either form
+void launch_polar_one(double* Y, int n, double tol, int maxiter, int* flags, double* qnrm,
+                      double* y1, double* y2, double* lt, double* sx, hipStream_t s);
 
 // out[4] = eigenvalue sum, theta, polar iterations, orthogonalization status
 void launch_wf_results(const double* scal, const int* flags, const int* info, double* out,

@@ -311,24 +311,19 @@ void launch_polar_init(int* flags, hipStream_t s) {
   hipLaunchKernelGGL(k_polar_init, dim3(1), dim3(64), 0, s, flags);
 }
 
-// q <- q + I (q held -x^T x), qnrm2 = ||q||_F; the step taken next:
-// Bjorck-Bowie if qnrm2 < 1, Higham otherwise; done once qnrm2 <= tol
-// (the loop test of src/Matrix.cpp:2458 for the following iteration)
-__global__ __launch_bounds__(1024) void k_polar_norm(double* __restrict__ q, int n, double tol,
-                                                     int* __restrict__ flags,
+// qnrm2 = ||q||_F from the npart partial sums of squares of q = I - x^T x; the
+// step taken next: Bjorck-Bowie if qnrm2 < 1, Higham otherwise; done once
+// qnrm2 <= tol (the loop test of src/Matrix.cpp:2458 for the following iteration)
+__global__ __launch_bounds__(1024) void k_polar_norm(const double* __restrict__ part, int npart,
+                                                     double tol, int* __restrict__ flags,
                                                      double* __restrict__ qnrm) {
   if (flags[0]) {
     if (threadIdx.x == 0) { flags[1] = 1; flags[2] = 1; }
     return;
   }
   double v[1] = {0.0};
-  const long nn = (long)n * n;
-  for (long i = threadIdx.x; i < nn; i += 1024) {
-    const long col = i / n, row = i - col * n;
-    const double x = q[i] + (row == col ? 1.0 : 0.0);
-    q[i] = x;
-    v[0] += x * x;
-  }
+#pragma unroll 4
+  for (int i = threadIdx.x; i < npart; i += 1024) v[0] += part[i];
   bsum<1>(v);
   if (threadIdx.x == 0) {
     const double qn = sqrt(v[0]);
@@ -340,76 +335,33 @@ __global__ __launch_bounds__(1024) void k_polar_norm(double* __restrict__ q, int
   }
 }
 
-void launch_polar_norm(double* q, int n, double tol, int* flags, double* qnrm, hipStream_t s) {
-  hipLaunchKernelGGL(k_polar_norm, dim3(1), dim3(1024), 0, s, q, n, tol, flags, qnrm);
-}
-
-__global__ __launch_bounds__(256) void k_ident_axpy(double* __restrict__ t,
-                                                    const double* __restrict__ q, int n,
-                                                    double a, const int* __restrict__ skip) {
-  if (*skip) return;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (long)n * n) return;
-  const long col = i / n, row = i - col * n;
-  t[i] = (row == col ? 1.0 : 0.0) + a * q[i];
-}
-
-void launch_ident_axpy(double* t, const double* q, int n, double a, const int* skip,
+void launch_polar_norm(const double* part, int npart, double tol, int* flags, double* qnrm,
                        hipStream_t s) {
-  const long nn = (long)n * n;
-  hipLaunchKernelGGL(k_ident_axpy, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, t, q, n,
-                     a, skip);
-}
-
-__global__ __launch_bounds__(256) void k_copy_if_not(double* __restrict__ dst,
-                                                     const double* __restrict__ src, long count,
-                                                     const int* __restrict__ skip) {
-  if (*skip) return;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < count) dst[i] = src[i];
-}
-
-void launch_copy_if_not(double* dst, const double* src, long count, const int* skip,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(k_copy_if_not, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s, dst,
-                     src, count, skip);
+  hipLaunchKernelGGL(k_polar_norm, dim3(1), dim3(1024), 0, s, part, npart, tol, flags, qnrm);
 }
 
 // pieces of the Higham step x <- (x + x^-T) / 2 (src/Matrix.cpp:2500-2513),
 // with x^-T = x (x^T x)^-1 from the device-wide Cholesky of x^T x:
-// g = transpose of a row-major lower inverse (so g^T g = (x^T x)^-1),
-// x = (x + z) / 2, and the singular flag from the factorization
+// g = transpose of L^-T (so g^T g = (x^T x)^-1) and the singular flag from the
+// factorization
 __global__ __launch_bounds__(256) void k_transpose_if(double* __restrict__ dst,
                                                       const double* __restrict__ src, int n,
-                                                      const int* __restrict__ skip) {
+                                                      long lds, const int* __restrict__ skip) {
   if (*skip) return;
   __shared__ double tile[32][33];
   const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
   const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;
   for (int j = ty; j < 32; j += 8)
-    if (by + j < n && bx + tx < n) tile[j][tx] = src[(long)(by + j) * n + bx + tx];
+    if (by + j < n && bx + tx < n) tile[j][tx] = src[(by + j) * lds + bx + tx];
   __syncthreads();
   for (int j = ty; j < 32; j += 8)
     if (bx + j < n && by + tx < n) dst[(long)(bx + j) * n + by + tx] = tile[tx][j];
 }
 
-void launch_transpose_if(double* dst, const double* src, int n, const int* skip, hipStream_t s) {
+void launch_transpose_if(double* dst, const double* src, int n, long lds, const int* skip,
+                         hipStream_t s) {
   hipLaunchKernelGGL(k_transpose_if, dim3((n + 31) / 32, (n + 31) / 32), dim3(256), 0, s, dst, src,
-                     n, skip);
-}
-
-__global__ __launch_bounds__(256) void k_higham_update(double* __restrict__ x,
-                                                       const double* __restrict__ z, long count,
-                                                       const int* __restrict__ skip) {
-  if (*skip) return;
-  const long i = (long)blockIdx.x * 256 + threadIdx.x;
-  if (i < count) x[i] = 0.5 * (x[i] + z[i]);
-}
-
-void launch_higham_update(double* x, const double* z, int n, const int* skip, hipStream_t s) {
-  const long nn = (long)n * n;
-  hipLaunchKernelGGL(k_higham_update, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, s, x, z,
-                     nn, skip);
+                     n, lds, skip);
 }
 
 __global__ void k_polar_singular(const int* __restrict__ info, int* __restrict__ flags) {
@@ -550,81 +502,101 @@ void launch_mix_dots(const double* fs, const int* st, int nmax, long m, double* 
   hipLaunchKernelGGL(k_mix_dots, dim3(MIX_BLOCKS), dim3(256), 0, s, fs, st, nmax, m, partial);
 }
 
+// LDS written by some lanes of one wave, before others of it read it
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // theta = sum over eigenpairs (w_k > 0) of (u_k.b / w_k) u_k: the AndersonMixer's
-// dsyev solve (src/AndersonMixer.cpp:113-157) with a cyclic Jacobi eigensolver
-__global__ __launch_bounds__(64) void k_mix_solve(const double* __restrict__ partial,
-                                                  const int* __restrict__ st, int anderson,
-                                                  double* __restrict__ theta) {
-  if (!st[3] || !anderson) return;
-  const int nv = st[1];
-  if (nv <= 0) return;
-  __shared__ double sums[MIX_NSUM];
-  const int t = threadIdx.x;
-  if (t < MIX_NSUM) {
-    double acc = 0.0;
-    for (int b = 0; b < MIX_BLOCKS; b++) acc += partial[(long)b * MIX_NSUM + t];
-    sums[t] = acc;
-  }
-  __syncthreads();
-  if (t != 0) return;
-  double a[MIX_NMAX * MIX_NMAX], u[MIX_NMAX * MIX_NMAX], w[MIX_NMAX], bb[MIX_NMAX];
-  const int n = nv;
-  {
-    int q = 0;
-    for (int i = 0; i < MIX_NMAX; i++)
-      for (int j = 0; j <= i; j++, q++)
-        if (i < n) { a[i + j * n] = sums[q]; a[j + i * n] = sums[q]; }
-    for (int i = 0; i < n; i++) bb[i] = sums[MIX_NA + i];
-  }
-  for (int i = 0; i < n; i++)
-    for (int j = 0; j < n; j++) u[i + j * n] = i == j ? 1.0 : 0.0;
+// dsyev solve (src/AndersonMixer.cpp:113-157) with a Jacobi eigensolver.  The
+// rotations' serial chain bounds it: a round rotates disjoint pairs (p, q) together,
+// 8 lanes to a pair and lane k to row or column k, with the matrix in LDS.  One
+// thread, one pair at a time and the matrix in scratch memory: 115 us, now 31.
+__device__ __forceinline__ void mix_theta(const double (&sums)[4][MIX_NSUM], int n,
+                                          double* __restrict__ theta) {
+  constexpr int M = MIX_NMAX;
+  __shared__ double a[M][M + 1], u[M][M + 1];
+  __shared__ double ub[M];
+  const int t = threadIdx.x & 63;
+  auto sum = [&](int q) { return (sums[0][q] + sums[1][q]) + (sums[2][q] + sums[3][q]); };
+  const int i = t >> 3, k = t & 7;
+  a[i][k] = i < n && k < n ? (k <= i ? sum(i * (i + 1) / 2 + k) : sum(k * (k + 1) / 2 + i)) : 0.0;
+  u[i][k] = i == k ? 1.0 : 0.0;
+  wave_sync();
+  const int m = n + (n & 1);             // players of a round-robin, m - 1 rounds
   for (int sweep = 0; sweep < 100; sweep++) {
-    double off = 0.0;
-    for (int i = 0; i < n; i++)
-      for (int j = i + 1; j < n; j++) off += a[i + j * n] * a[i + j * n];
+    double off = k > i ? a[i][k] * a[i][k] : 0.0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) off += __shfl_xor(off, o, 64);
     if (off < 1e-300) break;
-    for (int p = 0; p < n; p++)
-      for (int q = p + 1; q < n; q++) {
-        const double apq = a[p + q * n];
-        if (apq == 0.0) continue;
-        const double th = (a[q + q * n] - a[p + p * n]) / (2.0 * apq);
+    for (int r = 0; r < m - 1; r++) {
+      // pair i of this round (lanes past the pairs rotate nothing)
+      int p = i == 0 ? m - 1 : (r + i) % (m - 1), q = i == 0 ? r : (r - i + m - 1) % (m - 1);
+      if (p > q) { const int x = p; p = q; q = x; }
+      const bool on = i < m / 2 && q < n && a[p][q] != 0.0;
+      double cs = 1.0, sn = 0.0;
+      if (on) {
+        const double th = (a[q][q] - a[p][p]) / (2.0 * a[p][q]);
         const double tt = (th >= 0 ? 1.0 : -1.0) / (fabs(th) + sqrt(th * th + 1.0));
-        const double cs = 1.0 / sqrt(tt * tt + 1.0), sn = tt * cs;
-        for (int k = 0; k < n; k++) {
-          const double akp = a[k + p * n], akq = a[k + q * n];
-          a[k + p * n] = cs * akp - sn * akq;
-          a[k + q * n] = sn * akp + cs * akq;
-        }
-        for (int k = 0; k < n; k++) {
-          const double apk = a[p + k * n], aqk = a[q + k * n];
-          a[p + k * n] = cs * apk - sn * aqk;
-          a[q + k * n] = sn * apk + cs * aqk;
-        }
-        for (int k = 0; k < n; k++) {
-          const double ukp = u[k + p * n], ukq = u[k + q * n];
-          u[k + p * n] = cs * ukp - sn * ukq;
-          u[k + q * n] = sn * ukp + cs * ukq;
-        }
+        cs = 1.0 / sqrt(tt * tt + 1.0);
+        sn = tt * cs;
       }
+      wave_sync();
+      if (on) {
+        const double akp = a[k][p], akq = a[k][q];
+        a[k][p] = cs * akp - sn * akq;
+        a[k][q] = sn * akp + cs * akq;
+        const double ukp = u[k][p], ukq = u[k][q];
+        u[k][p] = cs * ukp - sn * ukq;
+        u[k][q] = sn * ukp + cs * ukq;
+      }
+      wave_sync();
+      if (on) {
+        const double apk = a[p][k], aqk = a[q][k];
+        a[p][k] = cs * apk - sn * aqk;
+        a[q][k] = sn * apk + cs * aqk;
+      }
+      wave_sync();
+    }
   }
   double wmax = -1e300;
-  for (int k = 0; k < n; k++) {
-    w[k] = a[k + k * n];
-    wmax = fmax(wmax, w[k]);
-  }
+  for (int j = 0; j < n; j++) wmax = fmax(wmax, a[j][j]);
   const double eig_ratio = 0.0;
-  for (int i = 0; i < n; i++) theta[i] = 0.0;
-  for (int k = 0; k < n; k++)
-    if (w[k] > eig_ratio * wmax) {
-      double ub = 0.0;
-      for (int j = 0; j < n; j++) ub += u[j + k * n] * bb[j];
-      for (int i = 0; i < n; i++) theta[i] += (ub / w[k]) * u[i + k * n];
-    }
+  if (t < n) {
+    double v = 0.0;
+    for (int j = 0; j < n; j++) v += u[j][t] * sum(MIX_NA + j);
+    ub[t] = a[t][t] > eig_ratio * wmax ? v / a[t][t] : 0.0;
+  }
+  wave_sync();
+  if (t < n) {
+    double v = 0.0;
+    for (int j = 0; j < n; j++) v += ub[j] * u[t][j];
+    theta[t] = v;
+  }
+}
+
+__global__ __launch_bounds__(256) void k_mix_solve(const double* __restrict__ partial,
+                                                   const int* __restrict__ st, int anderson,
+                                                   double* __restrict__ theta) {
+  if (!st[3] || !anderson) return;
+  const int n = st[1];
+  if (n <= 0) return;
+  __shared__ double sums[4][MIX_NSUM];
+  const int t = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  if (t < MIX_NSUM) {
+    double acc = 0.0;
+#pragma unroll 16
+    for (int b = wv; b < MIX_BLOCKS; b += 4) acc += partial[(long)b * MIX_NSUM + t];
+    sums[wv][t] = acc;
+  }
+  __syncthreads();
+  if (wv == 0) mix_theta(sums, n, theta);
 }
 
 void launch_mix_solve(const double* partial, const int* st, int anderson, double* theta,
                       hipStream_t s) {
-  hipLaunchKernelGGL(k_mix_solve, dim3(1), dim3(64), 0, s, partial, st, anderson, theta);
+  hipLaunchKernelGGL(k_mix_solve, dim3(1), dim3(256), 0, s, partial, st, anderson, theta);
 }
 
 // fbar = f_k - sum theta_i (f_k - f_i), xbar likewise (src/AndersonMixer.cpp:253-268);

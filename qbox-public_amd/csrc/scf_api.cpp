@@ -41,7 +41,7 @@ struct PolarWs {
   int* flags = nullptr;
   double* qnrm = nullptr;
   int alloc(qbg_ctx* c, Allocs& a, int n) {
-    const size_t n2 = (size_t)n * n;
+    const size_t n2 = polar_elems(n);
     int rc;
     if ((rc = a.get(c, &Q, n2)) || (rc = a.get(c, &T, n2)) || (rc = a.get(c, &QT, n2)) ||
         (rc = a.get(c, &XP, n2)) || (rc = a.get(c, &aug, 2 * n2)) || (rc = a.get(c, &flags, 8)) ||
@@ -51,39 +51,46 @@ struct PolarWs {
   }
 };
 
-// DoubleMatrix::polar (src/Matrix.cpp:2446-2517) as a fixed launch sequence:
-// maxiter rounds, each skipped on the device once converged
+// DoubleMatrix::polar (src/Matrix.cpp:2446-2517): one work-group's kernel, or a
+// fixed launch sequence of maxiter rounds, each skipped on the device once
+// converged
 int polar_enqueue(const PolarWs& w, double* Y, int n, double tol, int maxiter, double* W,
                   size_t wsize, hipStream_t s) {
+  if (n <= POLAR_ONE) {
+    launch_polar_one(Y, n, tol, maxiter, w.flags, w.qnrm, w.XP, w.Q, w.T, w.aug, s);
+    return QBG_OK;
+  }
   launch_polar_init(w.flags, s);
-  const long n2 = (long)n * n;
+  // sums of squares of q: in the partials' space, past those of the largest split
+  const int nb = split_blocks((long)n * n);
+  if ((size_t)nb + (size_t)n * n > wsize) return QBG_E_INVAL;
+  const size_t wl = wsize - nb;
   for (int it = 0; it < maxiter; it++) {
-    // q = I - Y^T Y
-    if (gemm_syrk(Y, n, n, n, -1.0, 0.0, w.Q, n, W, wsize, s, w.flags + 0)) return QBG_E_INVAL;
-    launch_polar_norm(w.Q, n, tol, w.flags, w.qnrm, s);
+    // q = I - Y^T Y, T = I + 3q/4
+    SplitEnd q;
+    q.delta = 1.0;
+    q.T = w.T;
+    q.part = W + wl;
+    if (gemm_syrk(Y, n, n, n, -1.0, 0.0, w.Q, n, W, wl, s, w.flags + 0, q)) return QBG_E_INVAL;
+    launch_polar_norm(q.part, nb, tol, w.flags, w.qnrm, s);
     // Bjorck-Bowie: Y <- Y (I + q/2 (I + 3q/4))
-    launch_ident_axpy(w.T, w.Q, n, 0.75, w.flags + 1, s);
-    if (gemm_nn_splitk(w.Q, n, w.T, n, n, n, n, w.QT, n, W, wsize, s, w.flags + 1))
+    SplitEnd half;
+    half.delta = 1.0;
+    if (gemm_nn_splitk(w.Q, n, w.T, n, n, n, n, w.QT, n, W, wl, s, w.flags + 1, 0.5, half))
       return QBG_E_INVAL;
-    launch_ident_axpy(w.T, w.QT, n, 0.5, w.flags + 1, s);
-    if (gemm_nn_splitk(Y, n, w.T, n, n, n, n, w.XP, n, W, wsize, s, w.flags + 1))
-      return QBG_E_INVAL;
-    launch_copy_if_not(Y, w.XP, n2, w.flags + 1, s);
+    if (gemm_nn_splitk(Y, n, w.QT, n, n, n, n, Y, n, W, wl, s, w.flags + 1)) return QBG_E_INVAL;
     // Higham: Y <- (Y + Y^-T) / 2, Y^-T = Y (Y^T Y)^-1 with Y^T Y = I - q
     // (reusing the Bjorck-Bowie buffers, idle in a Higham step)
-    double* M = w.T;
-    double* Linv = w.QT;
+    double* SX = w.aug;
+    double* P = w.T;
     double* G = w.XP;
-    double* P = w.aug;
-    double* Z = w.aug + n2;
-    launch_ident_axpy(M, w.Q, n, -1.0, w.flags + 2, s);
-    potrf_device(M, n, n, w.flags + 5, W, s, w.flags + 2);
-    trtri(M, n, n, Linv, s, w.flags + 2);
-    launch_transpose_if(G, Linv, n, w.flags + 2, s);
-    if (gemm_syrk(G, n, n, n, 1.0, 0.0, P, n, W, wsize, s, w.flags + 2)) return QBG_E_INVAL;
-    if (gemm_nn_splitk(Y, n, P, n, n, n, n, Z, n, W, wsize, s, w.flags + 2))
+    chol_inverse(SX, n, w.Q, w.flags + 5, W, s, w.flags + 2);
+    launch_transpose_if(G, SX + n, n, 2L * n, w.flags + 2, s);
+    if (gemm_syrk(G, n, n, n, 1.0, 0.0, P, n, W, wl, s, w.flags + 2)) return QBG_E_INVAL;
+    SplitEnd mean;
+    mean.beta = 0.5;
+    if (gemm_nn_splitk(Y, n, P, n, n, n, n, Y, n, W, wl, s, w.flags + 2, 0.5, mean))
       return QBG_E_INVAL;
-    launch_higham_update(Y, Z, n, w.flags + 2, s);
     launch_polar_singular(w.flags + 5, w.flags, s);
   }
   return QBG_OK;
@@ -106,9 +113,9 @@ struct qbg_wfstep {
   double param = 0.0;
   int ngw = 0, nst = 0;
   bool bands = false;     // created for a band set (qbg_wfstep_create_bands)
-  // nst x nst matrices: residual A, overlap S / Cholesky L, X = L^-T,
-  // B = c^T c_last, Y = L^-1 B (polar), Z = L^-T Q
-  double *A = nullptr, *S = nullptr, *X = nullptr, *B = nullptr, *Y = nullptr, *Z = nullptr;
+  // nst x nst matrices: residual A, B = c^T c_last, Y = L^-1 B (polar), Z = L^-T Q;
+  // 2 nst x nst: overlap S = L L^T on top of X = L^-T
+  double *A = nullptr, *S = nullptr, *B = nullptr, *Y = nullptr, *Z = nullptr;
   double *Tc = nullptr, *W = nullptr;    // 2 ngw x nst product; split-K partials
   size_t wsize = 0;
   double *cl = nullptr, *dl = nullptr;   // PSDA: previous bands and directions
@@ -141,10 +148,9 @@ int gram_enqueue(qbg_wfstep* w, double* c, int ldc, hipStream_t s) {
   const long K = 2L * w->ngw, ldc2 = 2L * ldc;
   const int n = w->nst;
   cleanup(c, ldc, n, s);
-  if (gemm_syrk(c, ldc2, n, K, 2.0, -1.0, w->S, n, w->W, w->wsize, s)) return QBG_E_INVAL;
-  potrf(w->S, n, n, w->info, s, w->W);
-  trtri(w->S, n, n, w->X, s);
-  gemm_nn_triu(c, ldc2, w->X, n, K, n, w->Tc, K, s);
+  if (gemm_syrk(c, ldc2, n, K, 2.0, -1.0, w->S, 2L * n, w->W, w->wsize, s)) return QBG_E_INVAL;
+  chol_inverse(w->S, n, nullptr, w->info, w->W, s);
+  gemm_nn_triu(c, ldc2, w->S + n, 2L * n, K, n, w->Tc, K, s);
   launch_copy_cols_if(c, ldc2, w->Tc, K, K, n, w->info, s);
   return QBG_OK;
 }
@@ -155,19 +161,20 @@ int ortho_align_enqueue(qbg_wfstep* w, double* c, int ldc, hipStream_t s) {
   const long K = 2L * w->ngw, ldc2 = 2L * ldc;
   const int n = w->nst;
   cleanup(c, ldc, n, s);
-  if (gemm_syrk(c, ldc2, n, K, 2.0, -1.0, w->S, n, w->W, w->wsize, s)) return QBG_E_INVAL;
-  potrf(w->S, n, n, w->info, s, w->W);
-  trtri(w->S, n, n, w->X, s);                       // X = L^-T (column major)
+  if (gemm_syrk(c, ldc2, n, K, 2.0, -1.0, w->S, 2L * n, w->W, w->wsize, s)) return QBG_E_INVAL;
+  chol_inverse(w->S, n, nullptr, w->info, w->W, s);
+  const double* X = w->S + n;                       // L^-T
+  const long ldx = 2L * n;
   if (gemm_tn_splitk(c, ldc2, w->cl, K, n, n, K, 2.0, -1.0, w->B, n, w->W, w->wsize,
                      QBG_PREC_FP64, s))
     return QBG_E_INVAL;
   // Y = X^T B = L^-1 B
-  if (gemm_tn_splitk(w->X, n, w->B, n, n, n, n, 1.0, 0.0, w->Y, n, w->W, w->wsize,
+  if (gemm_tn_splitk(X, ldx, w->B, n, n, n, n, 1.0, 0.0, w->Y, n, w->W, w->wsize,
                      QBG_PREC_FP64, s))
     return QBG_E_INVAL;
   int rc = polar_enqueue(w->pw, w->Y, n, 1.e-6, 20, w->W, w->wsize, s);
   if (rc) return rc;
-  if (gemm_nn_splitk(w->X, n, w->Y, n, n, n, n, w->Z, n, w->W, w->wsize, s))   // Z = L^-T Q
+  if (gemm_nn_splitk(X, ldx, w->Y, n, n, n, n, w->Z, n, w->W, w->wsize, s))   // Z = L^-T Q
     return QBG_E_INVAL;
   gemm_nn(c, ldc2, w->Z, n, K, n, n, w->Tc, K, 0, QBG_PREC_FP64, s);  // c Z
   launch_copy_cols_if(c, ldc2, w->Tc, K, K, n, w->info, s);
@@ -210,7 +217,7 @@ static int wfstep_create(qbg_ef* ef, int kind, double param, int nst, qbg_wfstep
   w->npart = psda_partials(w->ngw, w->nst);
   Allocs& a = w->mem;
   int rc;
-  if ((rc = a.get(c, &w->S, n2)) || (rc = a.get(c, &w->X, n2)) || (rc = a.get(c, &w->Tc, K * w->nst)) ||
+  if ((rc = a.get(c, &w->S, 2 * n2)) || (rc = a.get(c, &w->Tc, K * w->nst)) ||
       (rc = a.get(c, &w->W, w->wsize)) || (rc = a.get(c, &w->ekin, w->nst)) ||
       (rc = a.get(c, &w->dotp, w->nst)) || (rc = a.get(c, &w->scal, 4)) ||
       (rc = a.get(c, &w->bpart, band_partials(w->nst))) ||
