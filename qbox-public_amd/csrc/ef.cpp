@@ -121,7 +121,8 @@ static void ef_free(qbg_ef* e) {
                e->d_rhops, e->d_twnl, e->d_tau, e->d_b, e->d_sftab, e->d_sfac, e->d_vion,
                e->d_dvion, e->d_rhopst, e->d_sp_first, e->d_atom_sp, e->d_rhor, e->d_vxc,
                e->d_vr, e->d_rhog, e->d_rhoelg, e->d_rhogt, e->d_vlocal, e->d_occ, e->d_fesr,
-               e->d_fion, e->d_scal, e->d_partial, e->d_m_atom, e->d_m_twnl, e->d_m_l,
+               e->d_fion, e->d_scal, e->d_partial, e->d_partial_side, e->d_m_atom, e->d_m_twnl,
+               e->d_m_l,
                e->d_m_ipr, e->d_m_npr, e->d_m_stride, e->d_m_dbase, e->d_m_wt, e->d_dmat,
                e->d_a_m0, e->d_a_npr, e->d_a_stride, e->d_anl, e->d_fnl, e->d_fout, e->d_work,
                e->d_dtwnl, e->d_dt_off, e->d_sp_npr, e->d_fac2, e->b_anl, e->b_c32,
@@ -420,6 +421,10 @@ static bool kpoint_maps(const host::Basis& wb, const host::Basis& ub, std::vecto
   return true;
 }
 
+// coefficients of all bands and k-points from which an evaluation uses the
+// side stream, and up to which in FP64 (see ef_side_ok)
+constexpr long SIDE_MIN = 3L << 20, SIDE_MAX_FP64 = 32L << 20;
+
 // EnergyFunctional's constructor (src/EnergyFunctional.cpp:67-226) for one
 // k-point: kp null or 0 gives the real (Gamma) basis
 static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, double ecut,
@@ -685,6 +690,7 @@ static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, do
         (rc = dalloc(c, &e->d_rhogt, (size_t)2 * ngv)) || (rc = dalloc(c, &e->d_vlocal, (size_t)2 * ngv)) ||
         (rc = dalloc(c, &e->d_fesr, 3 * e->nat)) || (rc = dalloc(c, &e->d_fion, 3 * e->nat)) ||
         (rc = dalloc(c, &e->d_scal, S_COUNT)) || (rc = dalloc(c, &e->d_partial, e->partial_doubles)) ||
+        (rc = dalloc(c, &e->d_partial_side, e->partial_doubles)) ||
         (rc = dalloc(c, &e->d_anl, (size_t)2 * e->M * 2 * ngwm)) ||
         (rc = dalloc(c, &e->d_fnl, (size_t)2 * e->M * nst)) ||
         (rc = dalloc(c, &e->d_fout, (size_t)e->M * nst)) ||
@@ -763,6 +769,8 @@ static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, do
       delete e;
       return rc;
     }
+    // (here and not at the first evaluation, which may be beside another thread's capture)
+    if ((long)e->ngw_max * nst * nkp >= SIDE_MIN) (void)c->side_ready();
     *out = e;
     return QBG_OK;
   }
@@ -1415,26 +1423,22 @@ static int nl_bf16(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
   return QBG_OK;
 }
 
-// EnergyFunctional::energy (src/EnergyFunctional.cpp:397-1044): nspin 1,
-// Gamma, LDA.  energies (host, 14): ekin eps enl ehart ehart_e ehart_ep
-// ehart_p exc dxc esr eself ecoul etotal total_charge; fion (host, 3*nat)
-// species-major; sigma (host, 7x6: total, ekin, eps, enl, ehart, exc, esr).
-// reuse: the caller guarantees that c holds what the last update_density
-// read; H*psi then starts from the transforms update_density kept
-static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double* hpsi,
-                     int ldh, int compute_forces, int compute_stress, int prec,
-                     bool reuse = false) {
-  if (!e || !c || ldc < e->ngw_max) return QBG_E_INVAL;
+// In the split modes the forward z pass completes H*psi: it stores
+// 0.5 kpg2 c + the nonlocal part (FP32, from the NN product) + the local
+// part, so neither the kinetic pass nor the NN product touches H*psi
+static bool ef_fin(const qbg_ef* e, const double* c, int compute_hpsi, const double* hpsi,
+                   int prec) {
+  return (prec == QBG_PREC_BF16X3 || prec == QBG_PREC_BF16X2) && compute_hpsi && hpsi != c &&
+         !e->cplx && zfwd_fin_ok(e->gw);
+}
+
+// what the call computes that neither the density nor the potential enters:
+// the kinetic and the nonlocal part.  fin: see ef_fin
+static int ef_orbital(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double* hpsi,
+                      int ldh, int compute_forces, int compute_stress, int prec, bool fin) {
   qbg_ctx* ctx = e->ctx;
-  if (!e->have_vhxc) return ctx->fail(QBG_E_STATE, "energy before update_vhxc");
-  if (compute_hpsi && (!hpsi || ldh < e->ngw_max)) return QBG_E_INVAL;
-  if (compute_stress && !e->vhxc_stress)
-    return ctx->fail(QBG_E_STATE, "stress requested but update_vhxc ran without stress");
-  if (prec < QBG_PREC_FP64 || prec > QBG_PREC_BF16X2) return ctx->fail(QBG_E_INVAL, "energy: prec");
-  const int fprec = prec == QBG_PREC_FP64 ? QBG_PREC_FP64 : QBG_PREC_FP32;   // band FFTs
-  QBG_HIP(ctx, hipSetDevice(ctx->device));
   hipStream_t s = ctx->stream;
-  const int ngw = e->wb.size, nst = e->nst, M = e->M;
+  const int nst = e->nst;
   // kinetic energy and hpsi = 0.5 kpg2 c (this store replaces the clear of dwf);
   // in the split modes the same pass writes the FP32 copy of c for the GEMMs
   const bool split = prec == QBG_PREC_BF16X3 || prec == QBG_PREC_BF16X2;
@@ -1442,10 +1446,6 @@ static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, doub
     const int rc = bf16_ensure(e);
     if (rc) return rc;
   }
-  // in the split modes the forward z pass completes H*psi: it stores
-  // 0.5 kpg2 c + the nonlocal part (FP32, from the NN product) + the local
-  // part, so neither the kinetic pass nor the NN product touches H*psi
-  const bool fin = split && compute_hpsi && hpsi != c && !e->cplx && zfwd_fin_ok(e->gw);
   // the kinetic and nonlocal parts of each k-point (one pass for one
   // k-point; a set sums each k-point's weighted parts, src/EnergyFunctional.cpp:446-543, 703-716)
   const int nk = e->nkp;
@@ -1491,6 +1491,83 @@ static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, doub
     e->fion_keep = false;
     launch_kacc_sum(e->d_kacc, nk, e->d_scal + S_KIN, e->d_scal + S_ENL, e->d_scal + S_NLS, s);
   }
+  return nrc;
+}
+
+// Whether the call's kinetic and nonlocal part (ef_orbital) runs on the
+// context's side stream beside the transforms: its products leave the memory
+// idle that the transforms wait for, and its small kernels leave compute units
+// idle.  Below SIDE_MIN coefficients the two events cost more than that gives (0.3 M
+// coefficients in FP64: 209 us in order, 244 us beside; 1.8 M: 1232 and 1270); 4.8 M in
+// three k-points 1710 and 1552 us, 5.6 M in FP64 2560 and 2495, 7 M in BF16
+// parts 1420 and 1370, 27 M 5384 and 5140, 118 M 22.5 and 22.0 ms.  In FP64, whose
+// transforms and products both wait for the FP64 units, 118 M take 57.1 and 57.3 ms.
+static bool ef_side_ok(qbg_ef* e, const double* c, int ldc, int compute_hpsi, const double* hpsi,
+                       int ldh, int prec) {
+  qbg_ctx* ctx = e->ctx;
+  const long coefs = (long)e->ngw_max * e->nst * e->nkp;
+  if (coefs < SIDE_MIN || (prec == QBG_PREC_FP64 && coefs > SIDE_MAX_FP64)) return false;
+  if (ctx->prof || ctx->capturing || ctx->side_pending) return false;
+  // refused calls report as they do in order; nothing is left to time or allocate
+  if (!c || ldc < e->ngw_max || prec < QBG_PREC_FP64 || prec > QBG_PREC_BF16X2) return false;
+  if (compute_hpsi && (!hpsi || ldh < e->ngw_max)) return false;
+  const int fprec = prec == QBG_PREC_FP64 ? QBG_PREC_FP64 : QBG_PREC_FP32;
+  if (!grid_settled(e->gw, fprec)) return false;
+  const bool split = prec == QBG_PREC_BF16X3 || prec == QBG_PREC_BF16X2;
+  if (split && (!e->b_anl || (prec == QBG_PREC_BF16X2 && !e->bf_tuned))) return false;
+  // the transforms read c while the side stream writes hpsi
+  const long n = 2L * e->nst * e->nkp;
+  if (compute_hpsi && c < hpsi + n * ldh && hpsi < c + n * ldc) return false;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  return ctx->side && hipSetDevice(ctx->device) == hipSuccess &&
+         hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess &&
+         cap == hipStreamCaptureStatusNone;
+}
+
+// ef_orbital on the side stream, with partial sums of its own; what follows
+// on the context's stream joins before it uses the results
+static int ef_orbital_side(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double* hpsi,
+                           int ldh, int compute_forces, int compute_stress, int prec) {
+  SideScope side(e->ctx);
+  std::swap(e->d_partial, e->d_partial_side);
+  struct Back {
+    qbg_ef* e;
+    ~Back() { std::swap(e->d_partial, e->d_partial_side); }
+  } back{e};
+  return ef_orbital(e, c, ldc, compute_hpsi, hpsi, ldh, compute_forces, compute_stress, prec,
+                    ef_fin(e, c, compute_hpsi, hpsi, prec));
+}
+
+// EnergyFunctional::energy (src/EnergyFunctional.cpp:397-1044): nspin 1,
+// Gamma, LDA.  energies (host, 14): ekin eps enl ehart ehart_e ehart_ep
+// ehart_p exc dxc esr eself ecoul etotal total_charge; fion (host, 3*nat)
+// species-major; sigma (host, 7x6: total, ekin, eps, enl, ehart, exc, esr).
+// reuse: the caller guarantees that c holds what the last update_density
+// read; H*psi then starts from the transforms update_density kept
+// orbital_done: ef_orbital_side has run for this call
+static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double* hpsi,
+                     int ldh, int compute_forces, int compute_stress, int prec,
+                     bool reuse = false, bool orbital_done = false) {
+  if (!e || !c || ldc < e->ngw_max) return QBG_E_INVAL;
+  qbg_ctx* ctx = e->ctx;
+  if (!e->have_vhxc) return ctx->fail(QBG_E_STATE, "energy before update_vhxc");
+  if (compute_hpsi && (!hpsi || ldh < e->ngw_max)) return QBG_E_INVAL;
+  if (compute_stress && !e->vhxc_stress)
+    return ctx->fail(QBG_E_STATE, "stress requested but update_vhxc ran without stress");
+  if (prec < QBG_PREC_FP64 || prec > QBG_PREC_BF16X2) return ctx->fail(QBG_E_INVAL, "energy: prec");
+  const int fprec = prec == QBG_PREC_FP64 ? QBG_PREC_FP64 : QBG_PREC_FP32;   // band FFTs
+  QBG_HIP(ctx, hipSetDevice(ctx->device));
+  hipStream_t s = ctx->stream;
+  const int ngw = e->wb.size, nst = e->nst;
+  const bool fin = ef_fin(e, c, compute_hpsi, hpsi, prec);
+  SideJoin join(ctx);
+  int nrc = QBG_OK;
+  if (!orbital_done)
+    nrc = ef_side_ok(e, c, ldc, compute_hpsi, hpsi, ldh, prec)
+              ? ef_orbital_side(e, c, ldc, compute_hpsi, hpsi, ldh, compute_forces,
+                                compute_stress, prec)
+              : ef_orbital(e, c, ldc, compute_hpsi, hpsi, ldh, compute_forces, compute_stress,
+                           prec, fin);
   if (nrc) return nrc;
   if (compute_stress) {
     ctx->prof_begin(QBG_K_OTHER);
@@ -1532,6 +1609,7 @@ static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, doub
                                                  e->d_hpair + 4L * nu * q0, nu, fprec, nullptr);
           if (rc) return rc;
         }
+      ctx->join_side();
       ctx->prof_begin(QBG_K_OTHER);
       for (int ik = 0; ik < e->nkp; ik++) {
         if (ik > 0) kswap(e, e->kset[ik]);
@@ -1555,6 +1633,7 @@ static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, doub
         if (rc) return rc;
       }
       if (kept) e->xres_c = nullptr;
+      ctx->join_side();
       ctx->prof_begin(QBG_K_OTHER);
       launch_unfold_add(e->d_hpair, nu, nst, ngw, e->d_unfold, hpsi, ldh, s);
       ctx->prof_end();
@@ -1585,6 +1664,7 @@ static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, doub
     }
     if (kept) e->xres_c = nullptr;   // transformed in place: consumed
   }
+  ctx->join_side();
   if (compute_forces) {
     ctx->prof_begin(QBG_K_OTHER);
     const int nchunk = 64;
@@ -1675,9 +1755,12 @@ int qbg_ef_evaluate_async(qbg_ef* e, const double* c, int ldc, double* hpsi, int
     if (!e || !c) return QBG_E_INVAL;
     const int hp = (flags & QBG_EF_HPSI) != 0, fo = (flags & QBG_EF_FORCES) != 0,
               st = (flags & QBG_EF_STRESS) != 0;
-    int rc = ef_update_density(e, c, ldc, prec, hp != 0);
+    SideJoin join(e->ctx);
+    const bool side = ef_side_ok(e, c, ldc, hp, hpsi, ldh, prec);
+    int rc = side ? ef_orbital_side(e, c, ldc, hp, hpsi, ldh, fo, st, prec) : QBG_OK;
+    if (!rc) rc = ef_update_density(e, c, ldc, prec, hp != 0);
     if (!rc) rc = qbg_ef_update_vhxc(e, st);
-    if (!rc) rc = ef_launch(e, c, ldc, hp, hpsi, ldh, fo, st, prec, true);
+    if (!rc) rc = ef_launch(e, c, ldc, hp, hpsi, ldh, fo, st, prec, true, side);
     return rc;
   });
 }

@@ -41,6 +41,40 @@ hipEvent_t qbg_ctx::prof_event() {
   return e;
 }
 
+bool qbg_ctx::side_ready() {
+  if (side) return true;
+  if (!fork_ev && hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming) != hipSuccess)
+    fork_ev = nullptr;
+  if (!side_ev && hipEventCreateWithFlags(&side_ev, hipEventDisableTiming) != hipSuccess)
+    side_ev = nullptr;
+  if (!fork_ev || !side_ev ||
+      hipStreamCreateWithFlags(&side, hipStreamNonBlocking) != hipSuccess) {
+    (void)hipGetLastError();          // the caller goes on with one stream
+    side = nullptr;
+  }
+  return side != nullptr;
+}
+
+void qbg_ctx::join_side() {
+  if (!side_pending) return;
+  side_pending = false;
+  // (should the wait be refused, the host waits instead)
+  if (hipStreamWaitEvent(stream, side_ev, 0) != hipSuccess) (void)hipStreamSynchronize(side);
+}
+
+qbg::SideScope::SideScope(qbg_ctx* c_) : c(c_), main(c_->stream) {
+  if (hipEventRecord(c->fork_ev, main) != hipSuccess ||
+      hipStreamWaitEvent(c->side, c->fork_ev, 0) != hipSuccess)
+    (void)hipStreamSynchronize(main);
+  c->stream = c->side;
+}
+
+qbg::SideScope::~SideScope() {
+  c->stream = main;
+  c->side_pending = hipEventRecord(c->side_ev, c->side) == hipSuccess;
+  if (!c->side_pending) (void)hipStreamSynchronize(c->side);
+}
+
 void qbg_ctx::prof_begin(int kind) {
   if (!prof || capturing) return;
   Rec r{kind, prof_event(), prof_event()};
@@ -131,6 +165,9 @@ int qbg_finalize(qbg_ctx* c) {
   (void)hipEventDestroy(c->ev0);
   (void)hipEventDestroy(c->ev1);
   if (c->join_ev) (void)hipEventDestroy(c->join_ev);
+  if (c->fork_ev) (void)hipEventDestroy(c->fork_ev);
+  if (c->side_ev) (void)hipEventDestroy(c->side_ev);
+  if (c->side) (void)hipStreamDestroy(c->side);
   (void)hipStreamDestroy(c->stream);
   delete c;
   return QBG_OK;
@@ -717,6 +754,7 @@ int qbg::hpsi_resident(qbg_grid* g, const double* v, int nst, double* hpsi, int 
     PROF(QBG_K_YVMUL, ypass(g, prec, Y_VMUL, nb, v, nullptr, nullptr, nullptr, 1.0, s));
     PROF(QBG_K_XFWD, xfwd(g, prec, nb, s));
     const ZFin fb = fin ? fin_batch(fin, band0) : ZFin{};
+    g->ctx->join_side();               // what it adds to, or reads through fin
     PROF(QBG_K_ZFWD, zfwd(g, prec, Z_PAIR, OUT_ACCUM, hpsi + 2L * ldh * band0, 2L * ldh, ldh,
                           last_has2, nb, s, fin ? &fb : nullptr));
   }
@@ -739,6 +777,7 @@ int qbg::rs_mul_add_bands(qbg_grid* g, const double* v, const double* c, int ldc
     PROF(QBG_K_YVMUL, ypass(g, prec, Y_VMUL, nb, v, nullptr, nullptr, nullptr, 1.0, s));
     PROF(QBG_K_XFWD, xfwd(g, prec, nb, s));
     const ZFin fb = fin ? fin_batch(fin, band0) : ZFin{};
+    g->ctx->join_side();               // what it adds to, or reads through fin
     PROF(QBG_K_ZFWD, zfwd(g, prec, Z_PAIR, OUT_ACCUM, hpsi + 2L * ldh * band0, 2L * ldh, ldh,
                           last_has2, nb, s, fin ? &fb : nullptr));
   }

@@ -39,6 +39,14 @@ struct qbg_ctx {
   qbg_ctx* capture_origin = nullptr;
   hipEvent_t join_ev = nullptr;     // recorded by qbg_stream_join(this, ...)
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // a second stream for work that is independent of what stream does
+  // meanwhile, inside one call (SideScope): fork_ev orders it after what
+  // stream holds, side_ev stream after it (join_side)
+  hipStream_t side = nullptr;
+  hipEvent_t fork_ev = nullptr, side_ev = nullptr;
+  bool side_pending = false;        // side holds work that stream has not waited for
+  bool side_ready();                // creates them at the first use
+  void join_side();
   std::string err;
   // per-kernel event profiler
   bool prof = false;
@@ -56,6 +64,28 @@ struct qbg_ctx {
     return code;
   }
 };
+
+namespace qbg {
+// While it lives, c->stream is c->side, which starts after all that the
+// stream holds; its end records side_ev, which join_side makes the stream wait for.
+// c->side_ready() and no capture, event profile or pending side work before it.
+struct SideScope {
+  qbg_ctx* c;
+  hipStream_t main;
+  explicit SideScope(qbg_ctx* c_);
+  ~SideScope();
+  SideScope(const SideScope&) = delete;
+  SideScope& operator=(const SideScope&) = delete;
+};
+// joins on every way out of a call
+struct SideJoin {
+  qbg_ctx* c;
+  explicit SideJoin(qbg_ctx* c_) : c(c_) {}
+  ~SideJoin() { c->join_side(); }
+  SideJoin(const SideJoin&) = delete;
+  SideJoin& operator=(const SideJoin&) = delete;
+};
+}  // namespace qbg
 
 // column tile of the z pass: ncol workspace columns, the first np of them
 // at [col0, col0+np) (+G columns), the rest at [colm, colm+ncol-np) (-G
@@ -168,6 +198,8 @@ int grid_ensure_ws(qbg_grid* g, int npairs);
 // the fastest for prec (once per grid and precision; not while capturing;
 // the workspace must exist and holds no data across this call)
 int grid_tune(qbg_grid* g, int prec);
+// whether grid_tune has nothing left to time
+bool grid_settled(const qbg_grid* g, int prec);
 // bytes of one pair's x workspace at precision prec (both pass families)
 size_t xpair_bytes(const qbg_grid* g, int prec);
 // allocate the resident x array for npairs pairs (sized for FP64); returns

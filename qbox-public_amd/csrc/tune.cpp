@@ -144,9 +144,13 @@ int measure(qbg_grid* g, int prec, int pi, Choice* best) {
 
 }  // namespace
 
+bool grid_settled(const qbg_grid* g, int prec) {
+  return g->tuned[prec == QBG_PREC_FP64 ? 0 : 1] || !g->f4[0] || !g->f4[1];
+}
+
 int grid_tune(qbg_grid* g, int prec) {
   const int pi = prec == QBG_PREC_FP64 ? 0 : 1;
-  if (g->tuned[pi] || !g->f4[0] || !g->f4[1]) return QBG_OK;
+  if (grid_settled(g, prec)) return QBG_OK;
   if (g->ctx->capturing || !g->d_xbuf || !g->d_zbuf || g->ws_pairs < 1) return QBG_OK;
   int dev = g->ctx->device;
   const Key key{dev, g->np0, g->np1, g->np2, g->nact, g->ncols, pi, g->yppb_fixed ? g->yppb : 0};
