@@ -12,7 +12,7 @@
 // Same product shape as gemm.hip: D[p][q] = sum_r P(r,p) Q(r,q) on a
 // 128 x 128 tile per block of 256 threads (2 x 2 waves of 64 x 64), or, when
 // both output extents are multiples of 256 and NS = 2, a 256 x 256 tile per
-// block of 512 threads (k_gemm_bfb), with
+// block of 512 threads (k_gemm_bfd), with
 // P(r,p) = P[r + p*ldp] and Q(r,q) = Q[r + q*ldq] (TN) or Q[q + r*ldq] (NN).
 // All operand extents are padded (rows to BK, columns to the tile edge, leading
 // dimensions to multiples of 4) and the padding holds zeros, so loads need
@@ -37,7 +37,18 @@ namespace {
 
 constexpr int BT = 128;    // tile edge (p and q)
 constexpr int BK = 32;     // reduction chunk (one MFMA k-step)
-constexpr int LR = 40;     // LDS row pitch in bf16 (80 bytes: conflict-free 16-byte reads)
+constexpr int LR = BK;     // LDS row pitch in bf16 (64 bytes)
+
+// Position of reduction index k in row `row`: the row's four 16-byte chunks
+// are permuted by the row so that no access meets a bank twice.  16-byte reads of
+// a fragment (16 rows, one chunk per 16 lanes) are served in groups of 16 lanes that mix
+// two chunks, rows 0-3 and 12-15 of one and rows 4-11 of the next, which a
+// padded pitch does not spread: with 80 bytes a read took 12 cycles instead of 8,
+// a third of the LDS cycles (counted).  16-byte writes go in groups of 8 lanes, which
+// hold one chunk of 8 rows or the 4 chunks of 2 rows.
+__device__ __forceinline__ int lds_k(int row, int k) {
+  return (((k >> 3) ^ (row >> 1) ^ -((row >> 3) & 1)) & 3) << 3 | (k & 7);
+}
 
 // round-to-nearest-even bfloat16 bits of x; `back` is the value as FP32
 __device__ __forceinline__ unsigned short bf16_rne(float x, float& back) {
@@ -95,7 +106,7 @@ struct BfArgs {
   long ldo, sstride;
   int accumulate;
   int vec;             // out and ldo allow the 4-wide vector stores
-  // force epilogue (k_gemm_bfb with FE): D = Y(K, m) of the force product is
+  // force epilogue (k_gemm_bfd with FE): D = Y(K, m) of the force product is
   // not stored; fpart[(m*3 + j)*ntq + q tile] = sum over the tile's G of
   // gx_j(G) Im(conj(anl(m, G)) Y(m, G))
   const float* fa;     // anl, fa[q + m*lda_fa]
@@ -120,6 +131,11 @@ inline unsigned xcd_grid(BfArgs& g, int nblk) {
   return (unsigned)((nblk + 7) & ~7);
 }
 
+// Bound by the MFMAs and, between two barriers, by the conversions and LDS
+// traffic that the other block of the CU has to cover.  With lds_k and its writes
+// free of conflicts (they were a third of the LDS cycles): 256 bands x 512 projectors x 211 k in
+// 3 parts TN 315 -> 291 us (1.14 PFLOP/s), NN 397 -> 379; 128 x 256 x 109 k in 2 parts TN 51 -> 46,
+// NN 62 -> 60; 512 x 1024 x 461 k in 2 parts TN 2.03 -> 1.81 ms.
 template <int NS, bool QR, typename TO>
 __global__ __launch_bounds__(256) void k_gemm_bf(BfArgs g) {
   __shared__ __align__(16) unsigned short sP[NS][BT][LR];
@@ -134,26 +150,25 @@ __global__ __launch_bounds__(256) void k_gemm_bf(BfArgs g) {
   else { iq = tt % g.tq; ip = tt / g.tq; }
   const long p0 = (long)ip * BT, q0 = (long)iq * BT;
   const long rb = (long)split * g.rper, re = min(g.nr, rb + g.rper);
-  // staging: r-contiguous operands as (row = 16 rows per 16 lanes, 16 k at
-  // 16*((tid>>4)&1)): each 16-lane group writes 16 consecutive rows at one k
-  // offset, the pattern of the fragment reads (no bank conflicts), and lanes
-  // l, l+16 read the two halves of one 128-byte row segment;
-  // q-contiguous Q as (q = tid&127, 16 k at 16*(tid>>7))
-  const int srow = (tid & 15) | ((tid >> 5) << 4), sk = ((tid >> 4) & 1) * 16;
+  // staging: r-contiguous operands as 4 lanes on the 128 bytes of a row, 8 k
+  // each, rows srow and srow + 64; q-contiguous Q as (q = tid&127, 16 k at
+  // 16*(tid>>7))
+  const int srow = tid >> 2, sk = (tid & 3) * 8;
   const int qrow = QR ? srow : (tid & 127), qk = QR ? sk : (tid >> 7) * 16;
   const float* Pp = g.P + (p0 + srow) * g.ldp + sk;
   const float* Qp = QR ? g.Q + (q0 + srow) * g.ldq + sk : g.Q + q0 + qrow + (long)qk * g.ldq;
+  const long p64 = 64 * g.ldp, q64 = 64 * g.ldq;
   float pv[16], qv[16];
   auto load = [&](long r0) {
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const float4 t = *reinterpret_cast<const float4*>(Pp + r0 + 4 * i);
+      const float4 t = *reinterpret_cast<const float4*>(Pp + (i >> 1) * p64 + r0 + 4 * (i & 1));
       pv[4 * i] = t.x; pv[4 * i + 1] = t.y; pv[4 * i + 2] = t.z; pv[4 * i + 3] = t.w;
     }
     if (QR) {
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const float4 t = *reinterpret_cast<const float4*>(Qp + r0 + 4 * i);
+        const float4 t = *reinterpret_cast<const float4*>(Qp + (i >> 1) * q64 + r0 + 4 * (i & 1));
         qv[4 * i] = t.x; qv[4 * i + 1] = t.y; qv[4 * i + 2] = t.z; qv[4 * i + 3] = t.w;
       }
     } else {
@@ -161,23 +176,28 @@ __global__ __launch_bounds__(256) void k_gemm_bf(BfArgs g) {
       for (int i = 0; i < 16; i++) qv[i] = Qp[(r0 + i) * g.ldq];
     }
   };
+  // (rows 64 apart have the same permutation)
+  const int pw = lds_k(srow, sk);
+  const int qw0 = lds_k(qrow, qk), qw1 = QR ? qw0 : lds_k(qrow, qk + 8);
   auto store = [&]() {
     u16x8 h[NS];
-    split8<NS>(pv, h);
 #pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sP[s][srow][sk]) = h[s];
-    split8<NS>(pv + 8, h);
+    for (int i = 0; i < 2; i++) {
+      split8<NS>(pv + 8 * i, h);
 #pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sP[s][srow][sk + 8]) = h[s];
-    split8<NS>(qv, h);
+      for (int s = 0; s < NS; s++)
+        *reinterpret_cast<u16x8*>(&sP[s][srow + 64 * i][pw]) = h[s];
+    }
 #pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sQ[s][qrow][qk]) = h[s];
-    split8<NS>(qv + 8, h);
+    for (int i = 0; i < 2; i++) {
+      split8<NS>(qv + 8 * i, h);
 #pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sQ[s][qrow][qk + 8]) = h[s];
+      for (int s = 0; s < NS; s++)
+        *reinterpret_cast<u16x8*>(&sQ[s][QR ? srow + 64 * i : qrow][i ? qw1 : qw0]) = h[s];
+    }
   };
   const int wp = (w & 1) * 64, wq = (w >> 1) * 64;
-  const int fr = lane & 15, fk = (lane >> 4) * 8;
+  const int fr = lane & 15, fk = lds_k(fr, (lane >> 4) * 8);
   v4f acc[4][4];
 #pragma unroll
   for (int i = 0; i < 4; i++)
@@ -258,205 +278,21 @@ __global__ __launch_bounds__(256) void k_gemm_bf(BfArgs g) {
     }
 }
 
-// 256 x 256 tiles for large products: 512 threads = 8 waves of 128 (p) x 64
-// (q), so each staged operand row serves twice as many outputs as in the
-// 128 x 128 kernel (half the operand traffic from L2 and the LDS writes per
-// MFMA); fragments of P are read one 16-row group at a time to keep the
-// registers of 2 waves per SIMD
 constexpr int BB = 256;
-template <int NS, bool QR, typename TO, bool FE = false>
-__global__ __launch_bounds__(512) void k_gemm_bfb(BfArgs g) {
-  __shared__ __align__(16) unsigned short sP[NS][BB][LR];
-  __shared__ __align__(16) unsigned short sQ[NS][BB][LR];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int b = xcd_block(g.nblk);
-  if (b < 0) return;
-  const int ntile = g.tp * g.tq;
-  const int split = b / ntile, tt = b - split * ntile;
-  int ip, iq;
-  if (g.pfast) { ip = tt % g.tp; iq = tt / g.tp; }
-  else { iq = tt % g.tq; ip = tt / g.tq; }
-  const long p0 = (long)ip * BB, q0 = (long)iq * BB;
-  const long rb = (long)split * g.rper, re = min(g.nr, rb + g.rper);
-  const int srow = (tid & 15) | ((tid >> 5) << 4), sk = ((tid >> 4) & 1) * 16;
-  const int qrow = QR ? srow : (tid & 255), qk = QR ? sk : (tid >> 8) * 16;
-  const float* Pp = g.P + (p0 + srow) * g.ldp + sk;
-  const float* Qp = QR ? g.Q + (q0 + srow) * g.ldq + sk : g.Q + q0 + qrow + (long)qk * g.ldq;
-  float pv[16], qv[16];
-  auto load = [&](long r0) {
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const float4 t = *reinterpret_cast<const float4*>(Pp + r0 + 4 * i);
-      pv[4 * i] = t.x; pv[4 * i + 1] = t.y; pv[4 * i + 2] = t.z; pv[4 * i + 3] = t.w;
-    }
-    if (QR) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float4 t = *reinterpret_cast<const float4*>(Qp + r0 + 4 * i);
-        qv[4 * i] = t.x; qv[4 * i + 1] = t.y; qv[4 * i + 2] = t.z; qv[4 * i + 3] = t.w;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; i++) qv[i] = Qp[(r0 + i) * g.ldq];
-    }
-  };
-  auto store = [&]() {
-    u16x8 h[NS];
-    split8<NS>(pv, h);
-#pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sP[s][srow][sk]) = h[s];
-    split8<NS>(pv + 8, h);
-#pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sP[s][srow][sk + 8]) = h[s];
-    split8<NS>(qv, h);
-#pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sQ[s][qrow][qk]) = h[s];
-    split8<NS>(qv + 8, h);
-#pragma unroll
-    for (int s = 0; s < NS; s++) *reinterpret_cast<u16x8*>(&sQ[s][qrow][qk + 8]) = h[s];
-  };
-  const int wp = (w & 1) * 128, wq = (w >> 1) * 64;
-  const int fr = lane & 15, fk = (lane >> 4) * 8;
-  v4f acc[8][4];
-#pragma unroll
-  for (int i = 0; i < 8; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  load(rb);
-  for (long r0 = rb; r0 < re; r0 += BK) {
-    store();
-    __syncthreads();
-    if (r0 + BK < re) load(r0 + BK);
-    bf16x8 bq[NS][4];
-#pragma unroll
-    for (int s = 0; s < NS; s++)
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-        bq[s][j] = *reinterpret_cast<const bf16x8*>(&sQ[s][wq + 16 * j + fr][fk]);
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      bf16x8 a[NS];
-#pragma unroll
-      for (int s = 0; s < NS; s++)
-        a[s] = *reinterpret_cast<const bf16x8*>(&sP[s][wp + 16 * i + fr][fk]);
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        v4f c = acc[i][j];
-        if constexpr (NS == 3) {
-          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[0][j], a[2], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[1][j], a[1], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[2][j], a[0], c, 0, 0, 0);
-        }
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[0][j], a[1], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[1][j], a[0], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bq[0][j], a[0], c, 0, 0, 0);
-        acc[i][j] = c;
-      }
-    }
-    __syncthreads();
-  }
-  if constexpr (FE) {
-    // one projector fragment i at a time (3 double sums live): lane p =
-    // p0 + wp + 16 i + fr, G vectors ig, ig+1 of each q fragment (q even:
-    // re/im pairs); then the four lane groups sharing p, through LDS the
-    // four waves sharing wp
-    const int fq = 4 * (lane >> 4);
-    const int wg = w >> 1;
-    __syncthreads();                      // LDS tiles are free now
-    double* red = reinterpret_cast<double*>(&sP[0][0][0]);   // [4][256][3]
-    // the tile's G vectors q0/2 .. q0/2 + 127, staged once: gxs[c][ig - q0/2]
-    double* gxs = red + 4 * BB * 3;
-    for (int t = tid; t < 3 * (BB / 2); t += 512) {
-      const int c = t / (BB / 2), k = t - c * (BB / 2);
-      const long ig = (q0 >> 1) + k;
-      gxs[t] = ig < g.ngw ? g.gx[(long)c * g.ngw + ig] : 0.0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-      const long p = p0 + wp + 16 * i + fr;
-      double v0 = 0.0, v1 = 0.0, v2 = 0.0;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        const long q = q0 + wq + 16 * j + fq;
-        const int k = (int)((q - q0) >> 1);   // local G index (zero beyond ngw)
-        const float4 a = *reinterpret_cast<const float4*>(g.fa + q + p * g.lda_fa);
-        const double t0 = (double)a.y * acc[i][j][0] - (double)a.x * acc[i][j][1];
-        const double t1 = (double)a.w * acc[i][j][2] - (double)a.z * acc[i][j][3];
-        v0 += gxs[k] * t0 + gxs[k + 1] * t1;
-        v1 += gxs[BB / 2 + k] * t0 + gxs[BB / 2 + k + 1] * t1;
-        v2 += gxs[BB + k] * t0 + gxs[BB + k + 1] * t1;
-      }
-      v0 += __shfl_xor(v0, 16); v0 += __shfl_xor(v0, 32);
-      v1 += __shfl_xor(v1, 16); v1 += __shfl_xor(v1, 32);
-      v2 += __shfl_xor(v2, 16); v2 += __shfl_xor(v2, 32);
-      if (lane < 16) {
-        double* r = red + (wg * BB + wp + 16 * i + lane) * 3;
-        r[0] = v0; r[1] = v1; r[2] = v2;
-      }
-    }
-    __syncthreads();
-    for (int t = tid; t < BB * 3; t += 512) {
-      const int pl = t / 3, c = t - 3 * pl;
-      const long p = p0 + pl;
-      if (p < g.np) {
-        const double sum = ((red[(0 * BB + pl) * 3 + c] + red[(1 * BB + pl) * 3 + c]) +
-                            red[(2 * BB + pl) * 3 + c]) + red[(3 * BB + pl) * 3 + c];
-        g.fpart[(p * 3 + c) * g.ntq + iq] = sum;
-      }
-    }
-    return;
-  }
-  TO* o = (TO*)g.out + (long)split * g.sstride;
-  const int fq = 4 * (lane >> 4);
-#pragma unroll
-  for (int i = 0; i < 8; i++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const long p = p0 + wp + 16 * i + fr;
-      const long q = q0 + wq + 16 * j + fq;
-      if (p >= g.np) continue;
-      TO* d = o + q + p * g.ldo;
-      if (g.vec && q + 3 < g.nq) {
-        if constexpr (sizeof(TO) == 4) {
-          float4 v = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-          if (g.accumulate) {
-            const float4 u = *reinterpret_cast<const float4*>(d);
-            v.x += u.x; v.y += u.y; v.z += u.z; v.w += u.w;
-          }
-          *reinterpret_cast<float4*>(d) = v;
-        } else {
-          double2 v0 = {(double)acc[i][j][0], (double)acc[i][j][1]};
-          double2 v1 = {(double)acc[i][j][2], (double)acc[i][j][3]};
-          if (g.accumulate) {
-            const double2 u0 = *reinterpret_cast<const double2*>(d);
-            const double2 u1 = *reinterpret_cast<const double2*>(d + 2);
-            v0.x = u0.x + v0.x; v0.y = u0.y + v0.y;
-            v1.x = u1.x + v1.x; v1.y = u1.y + v1.y;
-          }
-          *reinterpret_cast<double2*>(d) = v0;
-          *reinterpret_cast<double2*>(d + 2) = v1;
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-          if (q + e < g.nq) {
-            const TO v = (TO)acc[i][j][e];
-            d[e] = g.accumulate ? (TO)(d[e] + v) : v;
-          }
-      }
-    }
-}
 
-// 256 x 256 tiles with the 2-part split and two LDS stages (160 KB): the
+// 256 x 256 tiles with the 2-part split for large products: 512 threads = 8
+// waves of 128 (p) x 64 (q), so each staged operand row serves twice as many outputs
+// as in the 128 x 128 kernel (half the operand traffic from L2 and the LDS writes
+// per MFMA); fragments of P are read one 16-row group at a time to keep the
+// registers of 2 waves per SIMD.  Two LDS stages (128 KB): the
 // loop computes step i from one stage while the split parts of step i+1,
 // loaded into registers during step i-1, go into the other stage and the
 // loads of step i+2 are issued; one barrier per step.  An r-contiguous
 // operand is loaded with eight consecutive lanes on the 128 contiguous bytes
 // of one row (4 k per lane, rows 64 apart per load), so each load touches 8
 // whole cache lines; Q along q (NN) as pairs of adjacent q (one 8-byte load
-// per lane and k row).  Otherwise as k_gemm_bfb (same fragments, MFMA
-// order, epilogues).
+// per lane and k row).  MFMA order as in k_gemm_bf.
+// 512 bands x 1024 projectors x 461336: NN 1.60 -> 1.55 ms with the permuted rows.
 template <bool QR, typename TO, bool FE = false>
 __global__ __launch_bounds__(512) void k_gemm_bfd(BfArgs g) {
   __shared__ __align__(16) unsigned short sm[2][2][2][BB][LR];   // [stage][P/Q][part][row][k]
@@ -505,29 +341,29 @@ __global__ __launch_bounds__(512) void k_gemm_bfd(BfArgs g) {
     for (int j = 0; j < 4; j++) {
       u16x4 hi, lo;
       split4(pv + 4 * j, hi, lo);
-      *reinterpret_cast<u16x4*>(&sm[st][0][0][lrow + 64 * j][lk]) = hi;
-      *reinterpret_cast<u16x4*>(&sm[st][0][1][lrow + 64 * j][lk]) = lo;
+      *reinterpret_cast<u16x4*>(&sm[st][0][0][lrow + 64 * j][lds_k(lrow, lk)]) = hi;
+      *reinterpret_cast<u16x4*>(&sm[st][0][1][lrow + 64 * j][lds_k(lrow, lk)]) = lo;
     }
     if (QR) {
 #pragma unroll
       for (int j = 0; j < 4; j++) {
         u16x4 hi, lo;
         split4(qv + 4 * j, hi, lo);
-        *reinterpret_cast<u16x4*>(&sm[st][1][0][lrow + 64 * j][lk]) = hi;
-        *reinterpret_cast<u16x4*>(&sm[st][1][1][lrow + 64 * j][lk]) = lo;
+        *reinterpret_cast<u16x4*>(&sm[st][1][0][lrow + 64 * j][lds_k(lrow, lk)]) = hi;
+        *reinterpret_cast<u16x4*>(&sm[st][1][1][lrow + 64 * j][lds_k(lrow, lk)]) = lo;
       }
     } else {
       u16x8 h[2];
       split8<2>(qv, h);
-      *reinterpret_cast<u16x8*>(&sm[st][1][0][qq][qk]) = h[0];
-      *reinterpret_cast<u16x8*>(&sm[st][1][1][qq][qk]) = h[1];
+      *reinterpret_cast<u16x8*>(&sm[st][1][0][qq][lds_k(qq, qk)]) = h[0];
+      *reinterpret_cast<u16x8*>(&sm[st][1][1][qq][lds_k(qq, qk)]) = h[1];
       split8<2>(qv + 8, h);
-      *reinterpret_cast<u16x8*>(&sm[st][1][0][qq + 1][qk]) = h[0];
-      *reinterpret_cast<u16x8*>(&sm[st][1][1][qq + 1][qk]) = h[1];
+      *reinterpret_cast<u16x8*>(&sm[st][1][0][qq + 1][lds_k(qq + 1, qk)]) = h[0];
+      *reinterpret_cast<u16x8*>(&sm[st][1][1][qq + 1][lds_k(qq + 1, qk)]) = h[1];
     }
   };
   const int wp = (w & 1) * 128, wq = (w >> 1) * 64;
-  const int fr = lane & 15, fk = (lane >> 4) * 8;
+  const int fr = lane & 15, fk = lds_k(fr, (lane >> 4) * 8);
   v4f acc[8][4];
 #pragma unroll
   for (int i = 0; i < 8; i++)
@@ -704,7 +540,7 @@ int tn_slots() {
   return cache[dev];
 }
 
-// blocks of k_gemm_bfb<2, true, float> the current device runs at once
+// blocks of k_gemm_bfd<true, float> the current device runs at once
 int tnb_slots() {
   static int cache[64] = {0};
   int dev = 0;
