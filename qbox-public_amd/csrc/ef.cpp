@@ -653,10 +653,10 @@ static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, do
     std::vector<double> g2iv(e->vb.g2i), giv(e->vb.gi);
     const long N = e->N;
     const size_t nbmax = (size_t)std::max<long>((N + 255) / 256, (ngv + 255) / 256);
-    e->partial_doubles = std::max<size_t>(nbmax * 18, (size_t)e->nat * 64 * 3 + 16);
-    e->partial_doubles = std::max<size_t>(e->partial_doubles, ((size_t)e->M * nst + 255) / 256 + 16);
+    e->partial_doubles = std::max<size_t>(nbmax * (18 + 4), (size_t)e->nat * 64 * 3 + 16);
     e->partial_doubles = std::max<size_t>(e->partial_doubles,
-                                          (size_t)((ngwm + 255) / 256) * ((nst + 31) / 32) * 8);
+                                          ((size_t)e->M * nst + 255) / 256 + 16 +
+                                              (size_t)((ngwm + 255) / 256) * ((nst + 31) / 32) * 8);
     e->partial_doubles = std::max<size_t>(e->partial_doubles, (size_t)nsp * NLS_CHUNKS_MAX * 6);
     // split-K partials of the fnl product: up to 40 splits of M x nst
     e->work_doubles = std::max<size_t>((size_t)1 << 22, (size_t)40 * e->M * nst);
@@ -959,8 +959,6 @@ static int ef_update_density(qbg_ef* e, const double* c, int ldc, int prec, bool
   QBG_HIP(ctx, hipSetDevice(ctx->device));
   hipStream_t s = ctx->stream;
   if (prec < QBG_PREC_FP64 || prec > QBG_PREC_BF16X2) return ctx->fail(QBG_E_INVAL, "prec");
-  fill_zero(e->d_rhor, e->N, s);
-  if (e->nspin == 2) fill_zero(e->d_rhor2, e->N, s);
   const int fprec = prec == QBG_PREC_FP64 ? QBG_PREC_FP64 : QBG_PREC_FP32;
   e->xres_c = nullptr;
   int pairs = 0;
@@ -989,7 +987,7 @@ static int ef_update_density(qbg_ef* e, const double* c, int ldc, int prec, bool
     // spin's bands of each k-point
     if (e->nkp > 1 && e->nspin == 1)
       rc = density_batches(e->gw, e->d_cpair, nu, 2 * nst * e->nkp, e->d_dfac, e->d_rhor, fprec,
-                           res, 0);
+                           true, res, 0);
     for (int ik = 0; ik < e->nkp && e->nkp > 1 && e->nspin == 2 && !rc; ik++)
       for (int sp = 0; sp < 2 && !rc; sp++) {
         int b0, nb, p0;
@@ -997,14 +995,18 @@ static int ef_update_density(qbg_ef* e, const double* c, int ldc, int prec, bool
         const int q0 = ik * nst + b0;   // the first pair of these bands
         if (nb > 0)
           rc = density_batches(e->gw, e->d_cpair + 4L * nu * q0, nu, 2 * nb, e->d_dfac + 2 * q0,
-                               sp == 0 ? e->d_rhor : e->d_rhor2, fprec, res, q0);
+                               sp == 0 ? e->d_rhor : e->d_rhor2, fprec, ik == 0, res, q0);
+        else if (ik == 0)
+          fill_zero(sp == 0 ? e->d_rhor : e->d_rhor2, e->N, s);
       }
     for (int sp = 0; sp < e->nspin && !rc && e->nkp == 1; sp++) {
       int b0, nb, p0;
       spin_bands(e, sp, b0, nb, p0);
       if (nb > 0)
         rc = density_batches(e->gw, e->d_cpair + 4L * nu * b0, nu, 2 * nb, e->d_dfac + 2 * b0,
-                             sp == 0 ? e->d_rhor : e->d_rhor2, fprec, res, b0);
+                             sp == 0 ? e->d_rhor : e->d_rhor2, fprec, true, res, b0);
+      else
+        fill_zero(sp == 0 ? e->d_rhor : e->d_rhor2, e->N, s);
     }
   }
   // one density per spin (src/ChargeDensity.cpp:136-160)
@@ -1013,7 +1015,9 @@ static int ef_update_density(qbg_ef* e, const double* c, int ldc, int prec, bool
     spin_bands(e, sp, b0, nb, p0);
     if (nb > 0)
       rc = density_batches(e->gw, c + 2L * ldc * b0, ldc, nb, e->d_dfac + 2 * p0,
-                           sp == 0 ? e->d_rhor : e->d_rhor2, fprec, res, p0);
+                           sp == 0 ? e->d_rhor : e->d_rhor2, fprec, true, res, p0);
+    else
+      fill_zero(sp == 0 ? e->d_rhor : e->d_rhor2, e->N, s);
   }
   if (rc) return rc;
   if (res) {
@@ -1063,14 +1067,17 @@ int qbg_ef_update_vhxc(qbg_ef* e, int compute_stress) {
     hipStream_t s = ctx->stream;
     ctx->prof_begin(QBG_K_OTHER);
     const double* rcore = e->core ? e->d_rhocr : nullptr;
+    int nl;
     if (e->nspin == 2)
-      launch_lsda(e->d_rhor, e->d_rhor2, rcore, e->N, e->d_vxc, e->d_vxc2, e->d_partial,
-                  e->d_scal + S_LDA, s);
+      nl = launch_lsda(e->d_rhor, e->d_rhor2, rcore, e->N, e->d_vxc, e->d_vxc2, e->d_partial, s);
     else
-      launch_lda(e->d_rhor, rcore, e->N, e->d_vxc, e->d_partial, e->d_scal + S_LDA, s);
-    launch_vhxc_g(e->d_rhog, e->vb.size, 1.0 / e->omega, e->d_vion, e->d_dvion, e->d_rhopst,
-                  e->d_g2iv, e->d_giv, e->d_gxv, e->d_rhoelg, e->d_rhogt, e->d_vlocal,
-                  compute_stress, e->d_partial, e->d_scal + S_VHXC, s);
+      nl = launch_lda(e->d_rhor, rcore, e->N, e->d_vxc, e->d_partial, s);
+    double* part2 = e->d_partial + 4L * nl;
+    const int nv = launch_vhxc_g(e->d_rhog, e->vb.size, 1.0 / e->omega, e->d_vion, e->d_dvion,
+                                 e->d_rhopst, e->d_g2iv, e->d_giv, e->d_gxv, e->d_rhoelg,
+                                 e->d_rhogt, e->d_vlocal, compute_stress, part2, s);
+    reduce_partials(Partials{e->d_partial, nl, 4, e->d_scal + S_LDA},
+                    Partials{part2, nv, 18, e->d_scal + S_VHXC}, s);
     ctx->prof_end();
     qbg_grid* g = e->gv;
     int rc = grid_ensure_ws(g, 1);
@@ -1126,12 +1133,30 @@ int qbg_ef_update_vhxc(qbg_ef* e, int compute_stress) {
   });
 }
 
+// fout = D fnl, enl, and the sums of both it and of the kin_blocks partial sums
+// that the kinetic pass left at d_partial, in one launch; W[n + m nst] = occw_n
+// fout[m, n] if W (the factor of the force product Y = c W)
+// (a launch of a few hundred threads takes 3 us here; an evaluation of 16 bands
+// went from 39 to 31 launches and from 207 to 189 us by this, the two density sums
+// in one, and outputs written by their first contribution instead of cleared)
+static void nl_enl(qbg_ef* e, const double* occ, int nst, const double* occw, double* W,
+                   int kin_blocks, hipStream_t s) {
+  double* part = e->d_partial + 8L * kin_blocks;
+  const int nb = launch_dmat_enl(e->d_fnl, e->M, nst, occ, e->d_m_ipr, e->d_m_npr, e->d_m_stride,
+                                 e->d_m_dbase, e->d_dmat, e->d_m_wt, 1.0 / e->omega, e->d_fout,
+                                 occw, W, part, s);
+  const Partials enl{part, nb, 1, e->o_enl};
+  if (kin_blocks) reduce_partials(Partials{e->d_partial, kin_blocks, 8, e->o_kin}, enl, s);
+  else reduce_partials(enl, Partials{}, s);
+}
+
 // EnergyFunctional::energy's nonlocal part (src/NonLocalPotential.cpp:1258-2069)
 // with the projector GEMMs on FP64 or FP32 MFMA (gemm.hip)
 // over the bands [b0, b0 + nst) of the functional (c and hpsi point at band
 // b0; their occupations are occ[b0 + n])
 static int nl_mfma(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double* hpsi, int ldh,
-                   int compute_forces, int compute_stress, int prec, int b0, int nst) {
+                   int compute_forces, int compute_stress, int prec, int b0, int nst,
+                   int kin_blocks) {
   qbg_ctx* ctx = e->ctx;
   hipStream_t s = ctx->stream;
   const int ngw = e->wb.size, M = e->M;
@@ -1159,9 +1184,11 @@ static int nl_mfma(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
   ctx->prof_end();
   if (grc) return ctx->fail(QBG_E_INVAL, "gemm workspace too small");
   ctx->prof_begin(QBG_K_NL);
-  launch_dmat_enl(e->d_fnl, M, nst, occ, e->d_m_ipr, e->d_m_npr, e->d_m_stride,
-                  e->d_m_dbase, e->d_dmat, e->d_m_wt, 1.0 / e->omega, e->d_fout, e->d_partial,
-                  e->o_enl, s);
+  // the force kernel's factor 4 is 2 (|F|^2) x 2 (G and -G); the full sphere
+  // of k != 0 takes half the occupation
+  const bool needy = compute_forces || compute_stress;
+  double* W = e->d_fnl + (size_t)M * nst;
+  nl_enl(e, occ, nst, e->cplx ? e->d_occh + b0 : occ, needy ? W : nullptr, kin_blocks, s);
   ctx->prof_end();
   if (compute_hpsi) {
     ctx->prof_begin(QBG_K_GEMM);
@@ -1169,19 +1196,11 @@ static int nl_mfma(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
     else gemm_nn(e->d_anl, K, e->d_fout, M, K, nst, M, hpsi, 2L * ldh, 1, prec, s);
     ctx->prof_end();
   }
-  if (compute_forces || compute_stress) {
+  if (needy) {
     // Y = c W with W[n,m] = occ_n fout[m,n] (stored in the second fnl block);
     // forces f_a,j = -4 sum_{m in a} sum_K (-i G_j anl)[K,m] Y[K,m] and the
     // nonlocal stress (src/NonLocalPotential.cpp:1786-2066) both reduce Y
-    double* W = e->d_fnl + (size_t)M * nst;
     void* Y = f32 ? (void*)(anl32 + (size_t)M * K) : (void*)(e->d_anl + (size_t)M * K);
-    ctx->prof_begin(QBG_K_NL);
-    if (compute_forces && !e->fion_keep)
-      fill_zero(e->d_fion, 3 * (size_t)e->nat, s);
-    // the force kernel's factor 4 is 2 (|F|^2) x 2 (G and -G); the full
-    // sphere of k != 0 takes half the occupation
-    launch_force_w(e->d_fout, e->cplx ? e->d_occh + b0 : occ, M, nst, W, s);
-    ctx->prof_end();
     ctx->prof_begin(QBG_K_GEMM);
     if (f32) gemm_nn(c, 2L * ldc, W, nst, K, M, nst, (float*)Y, K, 0, prec, s);
     else gemm_nn(c, 2L * ldc, W, nst, K, M, nst, (double*)Y, K, 0, prec, s);
@@ -1191,12 +1210,13 @@ static int nl_mfma(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
       // k != 0: the i anl half again, at its own column offset
       for (int half = 0; half < (e->cplx ? 2 : 1); half++) {
         const int32_t* am0 = half ? e->d_a_m0h : e->d_a_m0;
+        const int add = half || e->fion_keep;
         if (f32)
           launch_nl_forces_y(anl32, (const float*)Y, K, ngw, e->d_gxw, am0, e->d_a_npr,
-                             e->d_a_stride, e->nat, e->d_partial, 64, e->d_fion, s);
+                             e->d_a_stride, e->nat, e->d_partial, 64, e->d_fion, add, s);
         else
           launch_nl_forces_y(e->d_anl, (const double*)Y, K, ngw, e->d_gxw, am0, e->d_a_npr,
-                             e->d_a_stride, e->nat, e->d_partial, 64, e->d_fion, s);
+                             e->d_a_stride, e->nat, e->d_partial, 64, e->d_fion, add, s);
       }
     }
     if (compute_stress) {
@@ -1341,7 +1361,7 @@ static int bf16_tune(qbg_ef* e, const double* c, int ldc, int nst) {
 // instead of adding it to hpsi
 static int nl_bf16(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double* hpsi, int ldh,
                    int compute_forces, int compute_stress, int parts, bool c32_ready, int b0,
-                   int nst, float* yh = nullptr) {
+                   int nst, int kin_blocks, float* yh = nullptr) {
   qbg_ctx* ctx = e->ctx;
   hipStream_t s = ctx->stream;
   int rc = bf16_ensure(e);
@@ -1365,9 +1385,7 @@ static int nl_bf16(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
   ctx->prof_end();
   if (rc) return ctx->fail(QBG_E_INVAL, "bf16 gemm shape");
   ctx->prof_begin(QBG_K_NL);
-  launch_dmat_enl(e->d_fnl, M, nst, occ, e->d_m_ipr, e->d_m_npr, e->d_m_stride,
-                  e->d_m_dbase, e->d_dmat, e->d_m_wt, 1.0 / e->omega, e->d_fout, e->d_partial,
-                  e->o_enl, s);
+  nl_enl(e, occ, nst, nullptr, nullptr, kin_blocks, s);
   const bool needy = compute_forces || compute_stress;
   // W = occ fout for the force product (half the occupation on the full
   // sphere of k != 0, see nl_mfma)
@@ -1391,11 +1409,10 @@ static int nl_bf16(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
     ctx->prof_end();
     if (rc == 0) {
       ctx->prof_begin(QBG_K_NL);
-      if (!e->fion_keep) fill_zero(e->d_fion, 3 * (size_t)e->nat, s);
       for (int half = 0; half < (e->cplx ? 2 : 1); half++)
         launch_nl_forces_tiles(e->b_fpart, M, (int)(Kp / 256), e->b_fred,
                                half ? e->d_a_m0h : e->d_a_m0, e->d_a_npr, e->d_a_stride, e->nat,
-                               e->d_fion, s);
+                               e->d_fion, half || e->fion_keep, s);
       ctx->prof_end();
       return QBG_OK;
     }
@@ -1407,11 +1424,10 @@ static int nl_bf16(qbg_ef* e, const double* c, int ldc, int compute_hpsi, double
     if (rc) return ctx->fail(QBG_E_INVAL, "bf16 gemm shape");
     ctx->prof_begin(QBG_K_NL);
     if (compute_forces) {
-      if (!e->fion_keep) fill_zero(e->d_fion, 3 * (size_t)e->nat, s);
       for (int half = 0; half < (e->cplx ? 2 : 1); half++)
         launch_nl_forces_y(e->b_anl, (const float*)e->b_y32, Kp, ngw, e->d_gxw,
                            half ? e->d_a_m0h : e->d_a_m0, e->d_a_npr, e->d_a_stride, e->nat,
-                           e->d_partial, 64, e->d_fion, s);
+                           e->d_partial, 64, e->d_fion, half || e->fion_keep, s);
     }
     if (compute_stress)
       launch_nl_stress_y((const float*)e->b_y32, Kp, ngw, e->d_gxw, e->d_tau, e->nsp,
@@ -1469,19 +1485,19 @@ static int ef_orbital(qbg_ef* e, const double* c, int ldc, int compute_hpsi, dou
       launch_zero_rows_f32(e->b_c32, e->Kp, 2L * ngk, e->Kp, nst, s);
     // (the half sphere's G and -G times 1/2 is occ |c|^2 |G|^2; the full
     // sphere of k != 0 takes occ/2 |c|^2 |k+G|^2)
-    launch_kinetic(ck, ldc, nst, e->cplx ? e->d_occh : e->d_occ, ngk, e->d_g2w, e->d_gxw, hk,
-                   ldh, compute_hpsi && !fin, e->d_partial, e->o_kin, s,
-                   split ? e->b_c32 : nullptr, split ? e->Kp : 0);
+    const int kb = launch_kinetic(ck, ldc, nst, e->cplx ? e->d_occh : e->d_occ, ngk, e->d_g2w,
+                                  e->d_gxw, hk, ldh, compute_hpsi && !fin, e->d_partial, s,
+                                  split ? e->b_c32 : nullptr, split ? e->Kp : 0);
     ctx->prof_end();
     // nonlocal: anl, fnl = 2 anl^T c - anl0 c0^T (FP64 partial sums), the D
     // contraction and enl in FP64; in FP32 mode anl and Y are FP32 arrays and
     // the GEMMs run on FP32 MFMA; in the BF16 modes on the BF16-split path
     nrc = (prec == QBG_PREC_BF16X3 || prec == QBG_PREC_BF16X2)
               ? nl_bf16(e, ck, ldc, compute_hpsi, hk, ldh, compute_forces, compute_stress,
-                        prec == QBG_PREC_BF16X3 ? 3 : 2, true, 0, nst,
+                        prec == QBG_PREC_BF16X3 ? 3 : 2, true, 0, nst, kb,
                         fin ? e->b_yh : nullptr)
               : nl_mfma(e, ck, ldc, compute_hpsi, hk, ldh, compute_forces, compute_stress,
-                        prec, 0, nst);
+                        prec, 0, nst, kb);
     if (ik > 0) kswap(e, e->kset[ik]);
   }
   if (nk > 1) {
@@ -1676,10 +1692,9 @@ static int ef_launch(qbg_ef* e, const double* c, int ldc, int compute_hpsi, doub
   }
   // what this evaluation computed travels with its results, so a replayed
   // graph is read correctly after other evaluations ran in between
-  fill_value(e->d_scal + S_FLAGS, 1, compute_forces ? 1.0 : 0.0, s);
-  fill_value(e->d_scal + S_FLAGS + 1, 1, compute_stress ? 1.0 : 0.0, s);
-  // stage the scalars, G=0 values and forces in pinned host memory
-  gather_segments(e->d_seg_ptr, e->d_seg_n, 4, e->h_res, s);
+  // and stage the scalars, G=0 values and forces in pinned host memory
+  gather_segments(e->d_seg_ptr, e->d_seg_n, 4, e->h_res, s, e->d_scal + S_FLAGS,
+                  compute_forces ? 1.0 : 0.0, compute_stress ? 1.0 : 0.0);
   e->last_forces = compute_forces;
   e->last_stress = compute_stress;
   e->launched = 1;
@@ -1851,9 +1866,10 @@ int qbg_nl_energy(qbg_nl* nl, const double* c, int ldc, int compute_hpsi, double
     if (nb == 0) return QBG_OK;
     const int rc = (prec == QBG_PREC_BF16X3 || prec == QBG_PREC_BF16X2)
                        ? nl_bf16(e, c, ldc, compute_hpsi, dsd, ldd, compute_forces,
-                                 compute_stress, prec == QBG_PREC_BF16X3 ? 3 : 2, false, b0, nb)
+                                 compute_stress, prec == QBG_PREC_BF16X3 ? 3 : 2, false, b0, nb,
+                                 0)
                        : nl_mfma(e, c, ldc, compute_hpsi, dsd, ldd, compute_forces,
-                                 compute_stress, prec, b0, nb);
+                                 compute_stress, prec, b0, nb, 0);
     if (rc) return rc;
     hipStream_t s = ctx->stream;
     double sc[7];

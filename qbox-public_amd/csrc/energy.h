@@ -6,18 +6,27 @@
 
 namespace qbg {
 
+// nblocks x nv partial sums of a pass, and where their nv sums go
+struct Partials {
+  const double* partial = nullptr;
+  int nblocks = 0, nv = 0;
+  double* out = nullptr;
+};
+// two sets in one launch (b may be empty)
+void reduce_partials(const Partials& a, const Partials& b, hipStream_t s);
 void reduce_partials(const double* partial, int nblocks, int nv, double* out, hipStream_t s);
 
-// returns the number of partial blocks used (partial needs nb*8 doubles)
+// these four leave their partial sums (8, 4, 4 and 18 a block) to reduce_partials and
+// return the number of blocks
 int launch_kinetic(const double* c, long ldc, int nst, const double* occ, int ngw,
                    const double* g2, const double* gx, double* hpsi, long ldh, int store,
-                   double* partial, double* out8, hipStream_t s,
+                   double* partial, hipStream_t s,
                    float* c32 = nullptr, long ldk = 0);
 int launch_lda(const double* rho, const double* rc, long n, double* vxc, double* partial,
-               double* out4, hipStream_t s);
+               hipStream_t s);
 // spin-polarized LDA: vup, vdn and the same four partial sums as launch_lda
 int launch_lsda(const double* rup, const double* rdn, const double* rc, long n, double* vup,
-                double* vdn, double* partial, double* out4, hipStream_t s);
+                double* vdn, double* partial, hipStream_t s);
 // core density in G of the current structure factor, and the core term of dxc
 void launch_core_g(int ngv, int nsp, const double* sfac, const double* rhoc, double spin_fac,
                    double* rhocg, hipStream_t s);
@@ -27,7 +36,7 @@ void launch_lda_points(const double* rho, int n, double* e, double* v, hipStream
 int launch_vhxc_g(const double* rhog, int ngv, double omega_inv, const double* vion,
                   const double* dvion, const double* rhopst, const double* g2i, const double* gi,
                   const double* gx, double* rhoelg, double* rhogt, double* vlocal, int stress,
-                  double* partial, double* out18, hipStream_t s);
+                  double* partial, hipStream_t s);
 void launch_sf_tables(const double* tau, int nat, const double* b, const int* kmin, int krange,
                       double* tab, hipStream_t s);
 void launch_sfac(const int32_t* idx, int ngv, const double* tab, int krange, const int* kmin,
@@ -49,16 +58,15 @@ void launch_anl(int ngw, int nat, long lda, const double* gx, const double* tau,
                 const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
                 const int32_t* m_twnl, const int32_t* m_l, const double* twnl, void* A, int prec,
                 hipStream_t s);
+// enl as one partial sum a block (returns their number); W[n + m*nst] = occw_n fout if W
 int launch_dmat_enl(const double* F, int M, int nst, const double* occ, const int32_t* m_ipr,
                     const int32_t* m_npr, const int32_t* m_stride, const int32_t* m_dbase,
                     const double* dmat, const double* m_wt, double omega_inv, double* fout,
-                    double* partial, double* out1, hipStream_t s);
+                    const double* occw, double* W, double* partial, hipStream_t s);
 void launch_nl_forces(const double* fout, const double* dF, int M, int nst, const double* occ,
                       const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
                       int nat, double* fion, hipStream_t s);
 
-void launch_force_w(const double* fout, const double* occ, int M, int nst, double* W,
-                    hipStream_t s);
 // complex (k != 0) bands on a real band grid (kpoint.hip): each band n of c
 // (on S) to the pair (c1, c2) at columns 2n, 2n+1 of out (on U's half
 // sphere), and the pair transform's output back, added into hpsi
@@ -75,7 +83,8 @@ void launch_kacc_sum(const double* kacc, int nkp, double* kin, double* enl, doub
 template <typename T>
 void launch_nl_forces_y(const T* A, const T* Y, long lda, int ngw, const double* gx,
                         const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
-                        int nat, double* partial, int nchunk, double* fion, hipStream_t s);
+                        int nat, double* partial, int nchunk, double* fion, int add,
+                        hipStream_t s);
 
 // partial of launch_nl_stress_y: 6 nsp NLS_CHUNKS_MAX doubles
 constexpr int NLS_CHUNKS_MAX = 1024;
@@ -160,10 +169,10 @@ int gemm_bf_tn_default_split(int Mp, int Np, long Kp, int parts, int edge);
 int gemm_bf_nn_forces(const float* A, long lda, const float* F, long ldf, long Kp, int Np,
                       int Mp, int N, const float* anl, long lda_anl, const double* gx, int ngw,
                       double* fpart, hipStream_t s);
-// fion[3a+j] -= 4 sum over the atom's projectors and the ntq tiles of fpart
+// fion[3a+j] (or 0, unless add) - 4 sum over the atom's projectors and the ntq tiles of fpart
 void launch_nl_forces_tiles(const double* fpart, int M, int ntq, double* red,
                             const int32_t* a_m0, const int32_t* a_npr,
-                            const int32_t* a_stride, int nat, double* fion, hipStream_t s);
+                            const int32_t* a_stride, int nat, double* fion, int add, hipStream_t s);
 int gemm_bf_nn(const float* A, long lda, const float* F, long ldf, long Kp, int Np, int Mp,
                long K, int N, double* C, long ldc, int accumulate, int parts, hipStream_t s);
 int gemm_bf_nn(const float* A, long lda, const float* F, long ldf, long Kp, int Np, int Mp,

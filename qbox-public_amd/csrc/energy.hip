@@ -52,25 +52,29 @@ __device__ __forceinline__ void block_reduce_shfl(double (&v)[NV], double* __res
 }
 
 // out[q] = sum_b partial[b*nv + q] in block order; one block of 256 threads
-// per q-group, each thread summing a strided slice, then a tree.
-__global__ __launch_bounds__(256) void k_reduce_partials(const double* __restrict__ partial,
-                                                         int nblocks, int nv,
-                                                         double* __restrict__ out) {
+// per value of the two sets, each thread summing a strided slice, then a tree.
+__global__ __launch_bounds__(256) void k_reduce_partials(Partials s0, Partials s1) {
   __shared__ double red[256];
-  const int q = blockIdx.x;
+  const bool first = (int)blockIdx.x < s0.nv;
+  const Partials& p = first ? s0 : s1;
+  const int q = first ? blockIdx.x : blockIdx.x - s0.nv;
   double s = 0.0;
-  for (int b = threadIdx.x; b < nblocks; b += 256) s += partial[(long)b * nv + q];
+#pragma unroll 4
+  for (int b = threadIdx.x; b < p.nblocks; b += 256) s += p.partial[(long)b * p.nv + q];
   red[threadIdx.x] = s;
   __syncthreads();
   for (int st = 128; st > 0; st >>= 1) {
     if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[q] = red[0];
+  if (threadIdx.x == 0) p.out[q] = red[0];
 }
 
+void reduce_partials(const Partials& a, const Partials& b, hipStream_t s) {
+  hipLaunchKernelGGL(k_reduce_partials, dim3(a.nv + b.nv), dim3(256), 0, s, a, b);
+}
 void reduce_partials(const double* partial, int nblocks, int nv, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_reduce_partials, dim3(nv), dim3(256), 0, s, partial, nblocks, nv, out);
+  reduce_partials(Partials{partial, nblocks, nv, out}, Partials{}, s);
 }
 
 // ------------------------------------------------------- kinetic + ekin
@@ -115,11 +119,10 @@ __global__ __launch_bounds__(256) void k_kinetic(const double* __restrict__ c, l
 
 int launch_kinetic(const double* c, long ldc, int nst, const double* occ, int ngw,
                    const double* g2, const double* gx, double* hpsi, long ldh, int store,
-                   double* partial, double* out8, hipStream_t s, float* c32, long ldk) {
+                   double* partial, hipStream_t s, float* c32, long ldk) {
   const int nb = (ngw + 255) / 256, nch = (nst + KIN_BANDS - 1) / KIN_BANDS;
   hipLaunchKernelGGL(k_kinetic, dim3(nb, nch), dim3(256), 0, s, c, ldc, nst, occ, ngw, g2, gx,
                      hpsi, ldh, store, c32, ldk, partial);
-  reduce_partials(partial, nb * nch, 8, out8, s);
   return nb * nch;
 }
 
@@ -176,10 +179,9 @@ __global__ __launch_bounds__(256) void k_lda(const double* __restrict__ rho,
 }
 
 int launch_lda(const double* rho, const double* rc, long n, double* vxc, double* partial,
-               double* out4, hipStream_t s) {
+               hipStream_t s) {
   const int nb = (int)((n + 255) / 256);
   hipLaunchKernelGGL(k_lda, dim3(nb), dim3(256), 0, s, rho, rc, n, vxc, partial);
-  reduce_partials(partial, nb, 4, out4, s);
   return nb;
 }
 
@@ -256,10 +258,9 @@ __global__ __launch_bounds__(256) void k_lsda(const double* __restrict__ rup,
 }
 
 int launch_lsda(const double* rup, const double* rdn, const double* rc, long n, double* vup,
-                double* vdn, double* partial, double* out4, hipStream_t s) {
+                double* vdn, double* partial, hipStream_t s) {
   const int nb = (int)((n + 255) / 256);
   hipLaunchKernelGGL(k_lsda, dim3(nb), dim3(256), 0, s, rup, rdn, rc, n, vup, vdn, partial);
-  reduce_partials(partial, nb, 4, out4, s);
   return nb;
 }
 
@@ -323,11 +324,10 @@ __global__ __launch_bounds__(256) void k_vhxc_g(
 int launch_vhxc_g(const double* rhog, int ngv, double omega_inv, const double* vion,
                   const double* dvion, const double* rhopst, const double* g2i, const double* gi,
                   const double* gx, double* rhoelg, double* rhogt, double* vlocal, int stress,
-                  double* partial, double* out18, hipStream_t s) {
+                  double* partial, hipStream_t s) {
   const int nb = (ngv + 255) / 256;
   hipLaunchKernelGGL(k_vhxc_g, dim3(nb), dim3(256), 0, s, rhog, ngv, omega_inv, vion, dvion,
                      rhopst, g2i, gi, gx, rhoelg, rhogt, vlocal, stress, partial);
-  reduce_partials(partial, nb, 18, out18, s);
   return nb;
 }
 
@@ -649,7 +649,7 @@ void launch_anl(int ngw, int nat, long lda, const double* gx, const double* tau,
 // src/NonLocalPotential.cpp:1469-1571.  F (M x nst) holds fnl after the
 // G=0 correction and factor 2.  For column m (atom a, projector ipr of
 // species s): F'_m = sum_jpr D_s[ipr][jpr] F_{m(a,jpr)};
-// enl += occ_n wt/omega F F'; fout = wt/omega F'.
+// enl += occ_n wt/omega F F'; fout = wt/omega F'; if W, W[n + m*nst] = occw_n fout.
 // m_dbase[m]: offset of the species D block; m_npr[m]; m_stride[m] = na_s
 // (columns of one atom are ipr*na_s apart); m_ipr[m].
 __global__ __launch_bounds__(256) void k_dmat_enl(
@@ -657,7 +657,8 @@ __global__ __launch_bounds__(256) void k_dmat_enl(
     const int32_t* __restrict__ m_ipr, const int32_t* __restrict__ m_npr,
     const int32_t* __restrict__ m_stride, const int32_t* __restrict__ m_dbase,
     const double* __restrict__ dmat, const double* __restrict__ m_wt, double omega_inv,
-    double* __restrict__ fout, double* __restrict__ partial) {
+    double* __restrict__ fout, const double* __restrict__ occw, double* __restrict__ W,
+    double* __restrict__ partial) {
   const long t = (long)blockIdx.x * 256 + threadIdx.x;
   double v[1] = {0.0};
   if (t < (long)M * nst) {
@@ -670,6 +671,7 @@ __global__ __launch_bounds__(256) void k_dmat_enl(
     const double fac = m_wt[m] * omega_inv;
     v[0] = fac * occ[n] * F[t] * fp;
     fout[t] = fac * fp;
+    if (W) W[n + (long)m * nst] = occw[n] * (fac * fp);
   }
   block_reduce_store<1>(v, partial + blockIdx.x);
 }
@@ -677,12 +679,11 @@ __global__ __launch_bounds__(256) void k_dmat_enl(
 int launch_dmat_enl(const double* F, int M, int nst, const double* occ, const int32_t* m_ipr,
                     const int32_t* m_npr, const int32_t* m_stride, const int32_t* m_dbase,
                     const double* dmat, const double* m_wt, double omega_inv, double* fout,
-                    double* partial, double* out1, hipStream_t s) {
+                    const double* occw, double* W, double* partial, hipStream_t s) {
   const long tot = (long)M * nst;
   const int nb = (int)((tot + 255) / 256);
   hipLaunchKernelGGL(k_dmat_enl, dim3(nb), dim3(256), 0, s, F, M, nst, occ, m_ipr, m_npr,
-                     m_stride, m_dbase, dmat, m_wt, omega_inv, fout, partial);
-  reduce_partials(partial, nb, 1, out1, s);
+                     m_stride, m_dbase, dmat, m_wt, omega_inv, fout, occw, W, partial);
   return nb;
 }
 
@@ -722,20 +723,6 @@ void launch_nl_forces(const double* fout, const double* dF, int M, int nst, cons
 //         = -4 sum_{m in a} sum_K anl_j[K,m] Y[K,m],  Y = c W,  W[n,m] = occ_n fout[m,n],
 // with anl_j = -i G_j anl, i.e. in the real view anl_j[2ig] = G_j a_im,
 // anl_j[2ig+1] = -G_j a_re.  One GEMM instead of three.
-__global__ void k_force_w(const double* __restrict__ fout, const double* __restrict__ occ,
-                          int M, int nst, double* __restrict__ W) {
-  const long t = (long)blockIdx.x * 256 + threadIdx.x;
-  if (t >= (long)M * nst) return;
-  const int nb = (int)(t % nst), m = (int)(t / nst);
-  W[t] = occ[nb] * fout[m + (long)nb * M];     // W[nb + m*nst]
-}
-
-void launch_force_w(const double* fout, const double* occ, int M, int nst, double* W,
-                    hipStream_t s) {
-  const long tot = (long)M * nst;
-  hipLaunchKernelGGL(k_force_w, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s, fout, occ,
-                     M, nst, W);
-}
 
 // partial[(a*nchunk + chunk)*3 + j] = sum over the chunk's G and the atom's
 // projectors of G_j (a_im Y_re - a_re Y_im), accumulated in FP64 for FP32
@@ -767,14 +754,14 @@ __global__ __launch_bounds__(256) void k_nl_forces_y(
 // one block per atom, a wave each component: lanes take the chunks, then a
 // shuffle tree
 __global__ __launch_bounds__(192) void k_nl_forces_final(const double* __restrict__ partial,
-                                                         int nchunk,
-                                                         double* __restrict__ fion) {
+                                                         int nchunk, double* __restrict__ fion,
+                                                         int add) {
   const int a = blockIdx.x, j = threadIdx.x >> 6, lane = threadIdx.x & 63;
   double s = 0.0;
   for (int c = lane; c < nchunk; c += 64) s += partial[((long)a * nchunk + c) * 3 + j];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-  if (lane == 0) fion[3 * a + j] -= 4.0 * s;
+  if (lane == 0) fion[3 * a + j] = (add ? fion[3 * a + j] : 0.0) - 4.0 * s;
 }
 
 // the fused force product's partials: sum over the row tiles in a fixed-order
@@ -790,37 +777,40 @@ __global__ void k_nl_forces_proj(const double* __restrict__ red,
                                  const int32_t* __restrict__ a_m0,
                                  const int32_t* __restrict__ a_npr,
                                  const int32_t* __restrict__ a_stride, int nat,
-                                 double* __restrict__ fion) {
+                                 double* __restrict__ fion, int add) {
   const int t = blockIdx.x * 256 + threadIdx.x;
   if (t >= 3 * nat) return;
   const int a = t / 3, j = t - 3 * a;
   double sum = 0.0;
   for (int ip = 0; ip < a_npr[a]; ip++) sum += red[(long)(a_m0[a] + ip * a_stride[a]) * 3 + j];
-  fion[t] -= 4.0 * sum;
+  fion[t] = (add ? fion[t] : 0.0) - 4.0 * sum;
 }
 void launch_nl_forces_tiles(const double* fpart, int M, int ntq, double* red,
                             const int32_t* a_m0, const int32_t* a_npr,
-                            const int32_t* a_stride, int nat, double* fion, hipStream_t s) {
+                            const int32_t* a_stride, int nat, double* fion, int add,
+                            hipStream_t s) {
   hipLaunchKernelGGL(k_fpart_sum, dim3(3 * M), dim3(256), 0, s, fpart, ntq, red);
   hipLaunchKernelGGL(k_nl_forces_proj, dim3((3 * nat + 255) / 256), dim3(256), 0, s, red, a_m0,
-                     a_npr, a_stride, nat, fion);
+                     a_npr, a_stride, nat, fion, add);
 }
 
 template <typename T>
 void launch_nl_forces_y(const T* A, const T* Y, long lda, int ngw, const double* gx,
                         const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
-                        int nat, double* partial, int nchunk, double* fion, hipStream_t s) {
+                        int nat, double* partial, int nchunk, double* fion, int add,
+                        hipStream_t s) {
   const int chunk = (ngw + nchunk - 1) / nchunk;
   hipLaunchKernelGGL(k_nl_forces_y<T>, dim3(nchunk, nat), dim3(256), 0, s, A, Y, lda, ngw, gx, a_m0,
                      a_npr, a_stride, chunk, partial);
-  hipLaunchKernelGGL(k_nl_forces_final, dim3(nat), dim3(192), 0, s, partial, nchunk, fion);
+  hipLaunchKernelGGL(k_nl_forces_final, dim3(nat), dim3(192), 0, s, partial, nchunk, fion,
+                     add);
 }
 template void launch_nl_forces_y<double>(const double*, const double*, long, int, const double*,
                                          const int32_t*, const int32_t*, const int32_t*, int,
-                                         double*, int, double*, hipStream_t);
+                                         double*, int, double*, int, hipStream_t);
 template void launch_nl_forces_y<float>(const float*, const float*, long, int, const double*,
                                         const int32_t*, const int32_t*, const int32_t*, int,
-                                        double*, int, double*, hipStream_t);
+                                        double*, int, double*, int, hipStream_t);
 
 }  // namespace qbg
 

@@ -397,7 +397,8 @@ __global__ __launch_bounds__(256) void k_ypass(
       const int i = threadIdx.x + m * blockDim.x;
       if (i < nel) {
         const int j = i / nx, xl = i - j * nx;
-        rho[plane + (long)j * np0 + x0 + xl] += acc[m];
+        double* r = rho + plane + (long)j * np0 + x0 + xl;
+        *r = scale == 0.0 ? acc[m] : *r + acc[m];   // 0: written over what was there
       }
     }
   }

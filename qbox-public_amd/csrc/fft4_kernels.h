@@ -590,7 +590,11 @@ __global__ __launch_bounds__(xthreads(N1, N2)) void ky(
   }
   if (MC == 1 && vB) {
 #pragma unroll
-    for (int k2 = 0; k2 < N2; k2++) rho[plane + (long)Mp::out_b(q, k2) * np0 + x] += acc[k2 % NACC];
+    for (int k2 = 0; k2 < N2; k2++) {
+      // scale 0: the first batch of a density, written over what was there
+      double* r = rho + plane + (long)Mp::out_b(q, k2) * np0 + x;
+      *r = scale == 0.0 ? acc[k2 % NACC] : *r + acc[k2 % NACC];
+    }
   }
 }
 

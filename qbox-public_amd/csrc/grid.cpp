@@ -707,7 +707,7 @@ struct XwsScope {
 }  // namespace
 
 int qbg::density_batches(qbg_grid* g, const double* c, int ldc, int nst, const double* fac,
-                         double* rho, int prec, bool resident, int pair_base) {
+                         double* rho, int prec, bool clear, bool resident, int pair_base) {
   const int npairs = (nst + 1) / 2;
   const int B = std::min(npairs, g->batch);
   TRY(ensure_ws(g, B));
@@ -723,7 +723,8 @@ int qbg::density_batches(qbg_grid* g, const double* c, int ldc, int nst, const d
     XwsScope xs(g, resident ? (char*)g->d_xres + (size_t)(pair_base + p0) * pb : nullptr);
     PROF(QBG_K_ZBWD, zbwd(g, prec, Z_PAIR, c + 2L * ldc * band0, 2L * ldc, ldc, last_has2, nb, s));
     PROF(QBG_K_XBWD, xbwd(g, prec, nb, s));
-    PROF(QBG_K_YDENS, ypass(g, prec, Y_DENSITY, nb, nullptr, fac + 2 * p0, rho, nullptr, 1.0, s));
+    PROF(QBG_K_YDENS, ypass(g, prec, Y_DENSITY, nb, nullptr, fac + 2 * p0, rho, nullptr,
+                            clear && p0 == 0 ? 0.0 : 1.0, s));
   }
   return last_launch(g);
 }
@@ -855,7 +856,7 @@ int qbg_compute_density(qbg_grid* g, const double* c, int ldc, int nst, const do
     hipStream_t s = g->ctx->stream;
     QBG_HIP(g->ctx, hipMemcpyAsync(g->d_fac, fac.data(), sizeof(double) * fac.size(),
                                    hipMemcpyHostToDevice, s));
-    TRY(qbg::density_batches(g, c, ldc, nst, g->d_fac, rho, prec));
+    TRY(qbg::density_batches(g, c, ldc, nst, g->d_fac, rho, prec, false));
     // the host factor array must outlive the async copy
     QBG_HIP(g->ctx, hipStreamSynchronize(s));
     return QBG_OK;

@@ -42,10 +42,17 @@ void fill_value(double* p, size_t n, double v, hipStream_t s) {
 void fill_zero(double* p, size_t n, hipStream_t s) { fill_value(p, n, 0.0, s); }
 
 // gather scattered device scalars into one (host-mapped) buffer:
-// dst[i] = src segment by segment, segments (ptr, count) given in seg
+// dst[i] = src segment by segment, segments (ptr, count) given in seg;
+// before that flag[0] = f0, flag[1] = f1 (in one of the segments)
 __global__ __launch_bounds__(256) void k_gather(const double* const* __restrict__ seg_ptr,
                                                 const int* __restrict__ seg_n, int nseg,
-                                                double* __restrict__ dst) {
+                                                double* dst, double* flag, double f0,
+                                                double f1) {
+  if (threadIdx.x == 0) {
+    flag[0] = f0;
+    flag[1] = f1;
+  }
+  __syncthreads();
   int off = 0;
   for (int k = 0; k < nseg; k++) {
     const double* p = seg_ptr[k];
@@ -54,8 +61,8 @@ __global__ __launch_bounds__(256) void k_gather(const double* const* __restrict_
   }
 }
 void gather_segments(const double* const* seg_ptr, const int* seg_n, int nseg, double* dst,
-                     hipStream_t s) {
-  hipLaunchKernelGGL(k_gather, dim3(1), dim3(256), 0, s, seg_ptr, seg_n, nseg, dst);
+                     hipStream_t s, double* flag, double f0, double f1) {
+  hipLaunchKernelGGL(k_gather, dim3(1), dim3(256), 0, s, seg_ptr, seg_n, nseg, dst, flag, f0, f1);
 }
 
 // out[i] = a[i] + b[i]
