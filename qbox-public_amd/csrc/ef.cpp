@@ -656,7 +656,7 @@ static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, do
     e->partial_doubles = std::max<size_t>(nbmax * (18 + 4), (size_t)e->nat * 64 * 3 + 16);
     e->partial_doubles = std::max<size_t>(e->partial_doubles,
                                           ((size_t)e->M * nst + 255) / 256 + 16 +
-                                              (size_t)((ngwm + 255) / 256) * ((nst + 31) / 32) * 8);
+                                              kinetic_partials((int)ngwm, nst));
     e->partial_doubles = std::max<size_t>(e->partial_doubles, (size_t)nsp * NLS_CHUNKS_MAX * 6);
     // split-K partials of the fnl product: up to 40 splits of M x nst
     e->work_doubles = std::max<size_t>((size_t)1 << 22, (size_t)40 * e->M * nst);

@@ -18,6 +18,7 @@ void reduce_partials(const double* partial, int nblocks, int nv, double* out, hi
 
 // these four leave their partial sums (8, 4, 4 and 18 a block) to reduce_partials and
 // return the number of blocks
+size_t kinetic_partials(int ngw, int nst);   // doubles, for any basis up to ngw
 int launch_kinetic(const double* c, long ldc, int nst, const double* occ, int ngw,
                    const double* g2, const double* gx, double* hpsi, long ldh, int store,
                    double* partial, hipStream_t s,

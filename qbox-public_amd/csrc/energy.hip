@@ -81,20 +81,35 @@ void reduce_partials(const double* partial, int nblocks, int nv, double* out, hi
 // src/EnergyFunctional.cpp:441-571 (ekin, sigma_ekin) and :818-827
 // (cp += 0.5 kpg2 c); psi2sum(G) = sum_n occ_n |c_nG|^2 (fac = 1, real basis)
 // partial layout per block: [ekin, s_xx, s_yy, s_zz, s_xy, s_yz, s_xz, 0]
-// blockIdx.y: a chunk of KIN_BANDS bands (the sums below are linear in the
+// blockIdx.y: a chunk of `bands` bands (the sums below are linear in the
 // bands, so the chunks' partials add up); c32 (if given): the FP32 copy of
 // the coefficients for the split GEMMs, c32[2*ig + {0,1} + n*ldk], written in
 // the same pass over c
-constexpr int KIN_BANDS = 32;
+// Bound by HBM where there are blocks enough; a thread's serial walk over its
+// bands bounds the small calls, so the chunk shrinks from 32 bands to 4 until
+// KIN_BLOCKS blocks are there.  5.7 k x 16 bands 9.5 -> 5.7 us, 20 k x 90 26 -> 17,
+// 25 k x 64 34 -> 18 (22, 240 and 194 blocks of 32 bands before).
+constexpr int KIN_BLOCKS = 1024;
+static int kin_bands(int nb, int nst) {
+  int bands = 32;
+  while (bands > 4 && (long)nb * ((nst + bands - 1) / bands) < KIN_BLOCKS) bands /= 2;
+  return bands;
+}
+// halving the chunk at most doubles the blocks, from below KIN_BLOCKS (and adds
+// a block a column for an odd chunk count)
+size_t kinetic_partials(int ngw, int nst) {
+  const size_t nb = (ngw + 255) / 256;
+  return 8 * std::max(nb * ((nst + 31) / 32), (size_t)2 * KIN_BLOCKS + nb);
+}
 __global__ __launch_bounds__(256) void k_kinetic(const double* __restrict__ c, long ldc, int nst,
                                                  const double* __restrict__ occ, int ngw,
                                                  const double* __restrict__ g2,
                                                  const double* __restrict__ gx,
                                                  double* __restrict__ hpsi, long ldh, int store,
-                                                 float* __restrict__ c32, long ldk,
+                                                 float* __restrict__ c32, long ldk, int bands,
                                                  double* __restrict__ partial) {
   const int ig = blockIdx.x * 256 + threadIdx.x;
-  const int n0 = blockIdx.y * KIN_BANDS, n1 = min(nst, n0 + KIN_BANDS);
+  const int n0 = blockIdx.y * bands, n1 = min(nst, n0 + bands);
   double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (ig < ngw) {
     const double gg = g2[ig];
@@ -120,9 +135,10 @@ __global__ __launch_bounds__(256) void k_kinetic(const double* __restrict__ c, l
 int launch_kinetic(const double* c, long ldc, int nst, const double* occ, int ngw,
                    const double* g2, const double* gx, double* hpsi, long ldh, int store,
                    double* partial, hipStream_t s, float* c32, long ldk) {
-  const int nb = (ngw + 255) / 256, nch = (nst + KIN_BANDS - 1) / KIN_BANDS;
+  const int nb = (ngw + 255) / 256, bands = kin_bands(nb, nst);
+  const int nch = (nst + bands - 1) / bands;
   hipLaunchKernelGGL(k_kinetic, dim3(nb, nch), dim3(256), 0, s, c, ldc, nst, occ, ngw, g2, gx,
-                     hpsi, ldh, store, c32, ldk, partial);
+                     hpsi, ldh, store, c32, ldk, bands, partial);
   return nb * nch;
 }
 
@@ -590,8 +606,11 @@ void launch_local_forces(const int32_t* idx, int ngv, const double* tab, int kra
 // src/NonLocalPotential.cpp:1314-1395: anl = twnl (-i)^l e^{-iG.tau} for
 // l = 0, 1, 2.  One thread per (G, atom) forms the phase once and writes the
 // atom's projector columns m = a_m0[a] + ipr*a_stride[a]:
-// A[m*lda + 2*ig + {0,1}].
-constexpr int ANL_ATOMS = 8;
+// A[m*lda + 2*ig + {0,1}].  Bound by the stores; a thread takes up to ANL_ATOMS
+// atoms (G read once, their stores in flight together), fewer while there are not
+// ANL_BLOCKS blocks, where the serial walk over the atoms is what a call waits
+// for.  8 atoms x 5.7 k 13.5 -> 5.2 us, 40 x 20 k 18.5 -> 14.6.
+constexpr int ANL_ATOMS = 8, ANL_BLOCKS = 1024;
 template <typename T>
 struct alignas(2 * sizeof(T)) cpx2 {
   T x, y;
@@ -604,13 +623,12 @@ __global__ __launch_bounds__(256) void k_anl(int ngw, int nat, long lda, const d
                                              const int32_t* __restrict__ a_stride,
                                              const int32_t* __restrict__ m_twnl,
                                              const int32_t* __restrict__ m_l,
-                                             const double* __restrict__ twnl,
+                                             const double* __restrict__ twnl, int atoms,
                                              T* __restrict__ A) {
-  // ANL_ATOMS atoms per thread: G read once, the atoms' stores in flight
-  // together; each complex entry is one vector store
+  // each complex entry is one vector store
   const int ig = blockIdx.x * 256 + threadIdx.x;
   if (ig >= ngw) return;
-  const int a0 = blockIdx.y * ANL_ATOMS, a1 = min(nat, a0 + ANL_ATOMS);
+  const int a0 = blockIdx.y * atoms, a1 = min(nat, a0 + atoms);
   const double gxx = gx[ig], gyy = gx[ngw + ig], gzz = gx[2 * ngw + ig];
   for (int a = a0; a < a1; a++) {
     const double arg = -(gxx * tau[3 * a] + gyy * tau[3 * a + 1] + gzz * tau[3 * a + 2]);
@@ -636,13 +654,16 @@ void launch_anl(int ngw, int nat, long lda, const double* gx, const double* tau,
                 const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
                 const int32_t* m_twnl, const int32_t* m_l, const double* twnl, void* A, int prec,
                 hipStream_t s) {
-  dim3 grid((ngw + 255) / 256, (nat + ANL_ATOMS - 1) / ANL_ATOMS);
+  const int nb = (ngw + 255) / 256;
+  int atoms = ANL_ATOMS;
+  while (atoms > 1 && (long)nb * ((nat + atoms - 1) / atoms) < ANL_BLOCKS) atoms /= 2;
+  dim3 grid(nb, (nat + atoms - 1) / atoms);
   if (prec == 0)
     hipLaunchKernelGGL(k_anl<double>, grid, dim3(256), 0, s, ngw, nat, lda, gx, tau, a_m0,
-                       a_npr, a_stride, m_twnl, m_l, twnl, (double*)A);
+                       a_npr, a_stride, m_twnl, m_l, twnl, atoms, (double*)A);
   else
     hipLaunchKernelGGL(k_anl<float>, grid, dim3(256), 0, s, ngw, nat, lda, gx, tau, a_m0,
-                       a_npr, a_stride, m_twnl, m_l, twnl, (float*)A);
+                       a_npr, a_stride, m_twnl, m_l, twnl, atoms, (float*)A);
 }
 
 // ------------------------------------------------- D matrix, enl, forces
