@@ -422,8 +422,8 @@ static bool kpoint_maps(const host::Basis& wb, const host::Basis& ub, std::vecto
 }
 
 // coefficients of all bands and k-points from which an evaluation uses the
-// side stream, and up to which in FP64 (see ef_side_ok)
-constexpr long SIDE_MIN = 3L << 20, SIDE_MAX_FP64 = 32L << 20;
+// side stream, and up to which where the products are not split (see ef_side_ok)
+constexpr long SIDE_MIN = 3L << 20, SIDE_MAX_UNSPLIT = 32L << 20;
 
 // EnergyFunctional's constructor (src/EnergyFunctional.cpp:67-226) for one
 // k-point: kp null or 0 gives the real (Gamma) basis
@@ -1516,20 +1516,21 @@ static int ef_orbital(qbg_ef* e, const double* c, int ldc, int compute_hpsi, dou
 // idle.  Below SIDE_MIN coefficients the two events cost more than that gives (0.3 M
 // coefficients in FP64: 209 us in order, 244 us beside; 1.8 M: 1232 and 1270); 4.8 M in
 // three k-points 1710 and 1552 us, 5.6 M in FP64 2560 and 2495, 7 M in BF16
-// parts 1420 and 1370, 27 M 5384 and 5140, 118 M 22.5 and 22.0 ms.  In FP64, whose
-// transforms and products both wait for the FP64 units, 118 M take 57.1 and 57.3 ms.
+// parts 1420 and 1370, 27 M 5384 and 5140, 118 M 22.5 and 22.0 ms.  In FP64 and FP32,
+// whose long products keep most of the chip from the transforms, 27 M gain
+// 3 % and 118 M lose: 57.1 and 57.3 ms in FP64, 31.5 and 32.3 in FP32.
 static bool ef_side_ok(qbg_ef* e, const double* c, int ldc, int compute_hpsi, const double* hpsi,
                        int ldh, int prec) {
   qbg_ctx* ctx = e->ctx;
   const long coefs = (long)e->ngw_max * e->nst * e->nkp;
-  if (coefs < SIDE_MIN || (prec == QBG_PREC_FP64 && coefs > SIDE_MAX_FP64)) return false;
+  const bool split = prec == QBG_PREC_BF16X3 || prec == QBG_PREC_BF16X2;
+  if (coefs < SIDE_MIN || (!split && coefs > SIDE_MAX_UNSPLIT)) return false;
   if (ctx->prof || ctx->capturing || ctx->side_pending) return false;
   // refused calls report as they do in order; nothing is left to time or allocate
   if (!c || ldc < e->ngw_max || prec < QBG_PREC_FP64 || prec > QBG_PREC_BF16X2) return false;
   if (compute_hpsi && (!hpsi || ldh < e->ngw_max)) return false;
   const int fprec = prec == QBG_PREC_FP64 ? QBG_PREC_FP64 : QBG_PREC_FP32;
   if (!grid_settled(e->gw, fprec)) return false;
-  const bool split = prec == QBG_PREC_BF16X3 || prec == QBG_PREC_BF16X2;
   if (split && (!e->b_anl || (prec == QBG_PREC_BF16X2 && !e->bf_tuned))) return false;
   // the transforms read c while the side stream writes hpsi
   const long n = 2L * e->nst * e->nkp;
