@@ -336,9 +336,11 @@ constexpr double REDUCE_BYTES = 2000;    // bytes a cycle of the partials' store
 // (chunks) x (MFMA cycles of a wave's bi x bj blocks, 64 each in FP64, 32 in
 // FP32, and the chunk's fixed cost) + the traffic of the split partials.  It
 // makes the tiles follow ragged extents (131 bands: two 96-row tiles), and
-// small outputs use small tiles and many splits.  maxS: the most splits (1:
-// none); bjs: bit j allows bj = j; fixed bi, or 0; sym: square tiles, upper ones only.
-Pick pick(int np, int nq, long nr, long maxS, unsigned bjs, int bi_fixed, bool sym, int prec) {
+// small outputs use small tiles and many splits.  minS, maxS: the fewest and the
+// most splits (1, 1: none); bjs: bit j allows bj = j; fixed bi, or 0; sym: square tiles,
+// upper ones only.
+Pick pick(int np, int nq, long nr, long minS, long maxS, unsigned bjs, int bi_fixed, bool sym,
+          int prec) {
   const double cus = cu_count(), mf = prec == QBG_PREC_FP64 ? 256 : 128;
   const long chunks = (nr + KC - 1) / KC;
   Pick best{4, 4, 1};
@@ -351,7 +353,7 @@ Pick pick(int np, int nq, long nr, long maxS, unsigned bjs, int bi_fixed, bool s
       const long tq = (nq + 32 * bj - 1) / (32 * bj);
       const long tiles = sym ? tp * (tp + 1) / 2 : tp * tq;
       for (int k = 1; k <= 8; k++) {
-        long S = std::max<long>(1, (long)(k * cus) / tiles);
+        long S = std::max<long>(minS, (long)(k * cus) / tiles);
         S = std::min(S, std::min(maxS, std::max<long>(1, chunks / 2)));
         const double blocks = (double)tiles * S;
         const double rounds = blocks < 16 * cus ? (double)(((long)blocks + (long)cus - 1) /
@@ -369,6 +371,19 @@ Pick pick(int np, int nq, long nr, long maxS, unsigned bjs, int bi_fixed, bool s
     }
   }
   return best;
+}
+
+// The fewest splits of an FP32 product.  A split is one chain of FP32 sums
+// (the splits are added in FP64), whose rounding error grows as the square root
+// of its length, and the cycles alone would halve the splits where two blocks share
+// a CU anyway: 512 bands x 1024 projectors x 461 k in 16 splits, nonlocal H psi off by
+// 2.8e-6; in 32, 1.95e-6, for 1 % more of the product's time (its partials).  So a chain holds at
+// most a 1/32 of the reduction, or, of outputs of more than 32 tiles of 128 x 128, of
+// which 1024 blocks are enough, 1/(1024 / tiles); chains of 64 terms are
+// short enough for any.
+long fp32_splits(int np, int nq, long nr) {
+  const long tiles = (long)((np + 127) / 128) * ((nq + 127) / 128), chunks = (nr + KC - 1) / KC;
+  return std::max<long>(1, std::min(std::min<long>(32, (1024 + tiles - 1) / tiles), chunks / 4));
 }
 
 template <typename TPm, typename TQm, typename TC, bool QR, typename TO, int BI, int BJ>
@@ -408,7 +423,9 @@ int tn_splitk(const TQm* A, long lda, const double* B, long ldb, int M, int N, l
   g.np = N; g.nq = M; g.nr = K;
   g.pfast = 0;
   g.tri = sym ? 1 : 0;
-  const Pick k = pick(N, M, K, (long)(work_doubles / ((size_t)M * N)), BJ_TN, 0, sym != 0, prec);
+  const long minS = prec == QBG_PREC_FP64 ? 1 : fp32_splits(N, M, K);
+  const Pick k = pick(N, M, K, minS, (long)(work_doubles / ((size_t)M * N)), BJ_TN, 0, sym != 0,
+                      prec);
   const long chunks = (K + KC - 1) / KC;
   g.rper = ((chunks + k.S - 1) / k.S) * KC;
   const long S = (K + g.rper - 1) / g.rper;
@@ -439,7 +456,7 @@ void nn(const TQm* A, long lda, const double* F, long ldf, long K, int N, int M,
   g.tri = tri ? 2 : 0;
   g.rper = ((M + KC - 1) / KC) * KC;
   g.out = C; g.ldo = ldc; g.sstride = 0; g.accumulate = accumulate;
-  const Pick k = pick(N, (int)K, M, 1, BJ_NN, one_p ? (N + 31) / 32 : 0, false, prec);
+  const Pick k = pick(N, (int)K, M, 1, 1, BJ_NN, one_p ? (N + 31) / 32 : 0, false, prec);
   if constexpr (sizeof(TQm) == 8 && sizeof(TO) == 8) {
     if (prec == QBG_PREC_FP64) launch_gemm<double, TQm, double, false, TO>(g, k, s);
   }
@@ -463,7 +480,7 @@ int gemm_nn_splitk(const double* A, long lda, const double* F, long ldf, long K,
   g.pfast = 1;
   g.tri = 0;
   const long chunks = (M + KC - 1) / KC;
-  const Pick k = pick(N, (int)K, M, (long)(work_doubles / ((size_t)K * N)), BJ_NN, 0, false,
+  const Pick k = pick(N, (int)K, M, 1, (long)(work_doubles / ((size_t)K * N)), BJ_NN, 0, false,
                       QBG_PREC_FP64);
   g.rper = ((chunks + k.S - 1) / k.S) * KC;
   const long S = (M + g.rper - 1) / g.rper;

@@ -82,3 +82,36 @@ def test_nonlocal_products_ragged(ctx, oracle_mod, prec, na, nst):
     assert np.abs(r["fion"] - fref).max() < ftol * fs
     assert np.abs(h - ref["hpsi"]).max() < htol * np.abs(ref["hpsi"]).max()
     ef.release()
+
+
+def test_fp32_chain_length(ctx):
+    """The nonlocal H psi of FP32 products at a long reduction (K = 108672), whose
+    error is that of its chains of FP32 sums.  Adding term k rounds a partial sum of
+    variance k; the mean square of that, relative to the sum, is 2^-46 / 12 times the
+    mean of 1 / m^2 over the leading digits m (0.54), so a chain of n terms is off by
+    sqrt(0.045 / 2) 2^-23 sqrt(n) = 0.15 2^-23 sqrt(n), and a sum of independent
+    chains of that length by the same.  The projections may use chains of K / 32 terms
+    (the splits are added in FP64), the product with the projectors has M: 10 % above
+    both is 1.26e-6, and 1.08e-6 is measured; projections in chains of twice that
+    length take it to 1.43e-6."""
+    import qbg
+    nst = 300
+    s = cf.SystemDef("long reduction", np.diag([24.0, 24.0, 24.0]), 60.0, [cf.SPECIES_A], [175],
+                     nst, 77, 1.6).build_positions()
+    print(f"[case] {s.name}", flush=True)
+    ef = qbg.EnergyFunctional(ctx, s)
+    nl = qbg.NonLocalPotential(ef)
+    rng = np.random.default_rng(3)
+    c = rng.standard_normal((nst, ef.ngw)) + 1j * rng.standard_normal((nst, ef.ngw))
+    c[:, 0] = c[:, 0].real
+    dc, h = ctx.to_device(c), {}
+    for prec in ("fp64", "fp32"):
+        dh = ctx.to_device(np.zeros_like(c))
+        nl.energy(dc, dh, prec=prec)
+        h[prec] = dh.download()
+        dh.release()
+    err = np.linalg.norm(h["fp32"] - h["fp64"]) / np.linalg.norm(h["fp64"])
+    assert err < 1.1 * 0.15 * 2.0 ** -23 * np.sqrt(2 * ef.ngw / 32 + 4 * s.nat), err
+    dc.release()
+    nl.release()
+    ef.release()
