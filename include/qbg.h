@@ -124,10 +124,10 @@ int qbg_grid_info(const qbg_grid* g, int* out);
  * FFTW_MEASURE planning (src/FourierTransform.cpp:45-54, 830-1062).  At the
  * first batched call of a grid in a precision (compute_density, rs_mul_add,
  * the energy functional's passes), outside graph capture, the library times
- * every compiled line split of np0 (x pass) and np1 (y pass) and the y
- * pass's band pairs per block (8, 16, 32) on the grid's own workspace, keeps
- * the fastest, and caches the choice per device, grid shape and precision
- * for the process.  qbg_grid_tuning reports it: out[0] 1 once tuned for prec
+ * the compiled line splits of np0 (x pass) and np1 (y pass), except slower
+ * ones that only plans name, and the y pass's band pairs per block (8, 16,
+ * 32) on the grid's own workspace, keeps the fastest, and caches the choice
+ * per device, grid shape and precision for the process.  qbg_grid_tuning reports it: out[0] 1 once tuned for prec
  * (FP64, or any of the FP32-FFT modes), out[1..2] the x split n1 x n2,
  * out[3..4] the y split, out[5] the pairs per block (6 ints).
  * qbg_grid_plan fixes the choice instead (FFTW_ESTIMATE-like): x_n1, y_n1

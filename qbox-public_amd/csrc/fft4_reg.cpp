@@ -1,6 +1,7 @@
 // fft4_reg.cpp -- registry of the compiled four-step line lengths: the
-// default split of each length (fft4_a..d, fft4_g..o) and the alternatives the
-// grid's tuner may pick instead (fft4_e, fft4_f).
+// default split of each length (fft4_a..d, fft4_g..o), the alternatives the
+// grid's tuner may pick instead (fft4_e, fft4_f), and slower ones that callers' plans
+// may hold (fft4_p).
 //
 // Every even length 16 <= n <= 396 that Basis and ChargeDensity can choose
 // for a grid (2^a 3^b 5^c 7^d 11^e with b <= 2 and c, d, e <= 1, a >= 1) is
@@ -39,13 +40,16 @@ const F4Ops* f4_table_l(int* count);
 const F4Ops* f4_table_m(int* count);
 const F4Ops* f4_table_n(int* count);
 const F4Ops* f4_table_o(int* count);
+const F4Ops* f4_table_p(int* count);
 
 namespace {
 // defaults first, so the first match of a length is its default split
 const F4Ops* (*const kTables[])(int*) = {f4_table_a, f4_table_b, f4_table_c,
                                           f4_table_d, f4_table_g, f4_table_h, f4_table_i,
                                           f4_table_j, f4_table_k, f4_table_l, f4_table_m,
-                                          f4_table_n, f4_table_o, f4_table_e, f4_table_f};
+                                          f4_table_n, f4_table_o, f4_table_e, f4_table_f,
+                                          f4_table_p};
+constexpr int KEPT = 1;     // of them, at the end: not timed
 }  // namespace
 
 const F4Ops* f4_ops(int n) {
@@ -53,11 +57,12 @@ const F4Ops* f4_ops(int n) {
   return f4_candidates(n, &out, 1) ? out : nullptr;
 }
 
-int f4_candidates(int n, const F4Ops** out, int cap) {
+int f4_candidates(int n, const F4Ops** out, int cap, bool kept) {
+  const int tables = (int)(sizeof(kTables) / sizeof(kTables[0])) - (kept ? 0 : KEPT);
   int k = 0;
-  for (auto table : kTables) {
+  for (int j = 0; j < tables; j++) {
     int cnt = 0;
-    const F4Ops* t = table(&cnt);
+    const F4Ops* t = kTables[j](&cnt);
     for (int i = 0; i < cnt; i++)
       if (t[i].n == n && k < cap) out[k++] = &t[i];
   }

@@ -123,8 +123,9 @@ struct F4Ops {
                 const double* fac, double* rho, double* fgrid, double scale, hipStream_t s);
 };
 const F4Ops* f4_ops(int n);   // default split of n, nullptr if n has no compiled kernels
-// every compiled split of n (default first), at most cap; returns the count
-int f4_candidates(int n, const F4Ops** out, int cap);
+// the splits of n that the tuner times (default first), at most cap; returns the
+// count.  kept: and those that only qbg_grid_plan takes, after them
+int f4_candidates(int n, const F4Ops** out, int cap, bool kept = false);
 }  // namespace qbg
 
 struct qbg_grid {

@@ -1,8 +1,8 @@
 // tune.cpp -- launch tuner of a grid's batched FFT passes.
 //
 // At the first batched transform of a grid in a precision, outside graph
-// capture, the x-pass kernels of every compiled split of np0 and the y-pass
-// kernels of every compiled split of np1 (with 8, 16 and 32 band pairs per
+// capture, the x-pass kernels of the splits of np0 and the y-pass kernels of
+// those of np1 that f4_candidates lists (with 8, 16 and 32 band pairs per
 // block for the potential multiply) are timed on the grid's own workspace
 // and maps, with HIP events on the context's stream, and the fastest are
 // kept for that precision.  The choice is cached per device, grid shape and
@@ -205,7 +205,7 @@ extern "C" int qbg_grid_plan(qbg_grid* g, int prec, int x_n1, int y_n1, int yppb
     auto pick = [](int n, int n1, const qbg::F4Ops* dflt) -> const qbg::F4Ops* {
       if (n1 == 0) return dflt;
       const qbg::F4Ops* c[8];
-      const int k = qbg::f4_candidates(n, c, 8);
+      const int k = qbg::f4_candidates(n, c, 8, true);
       for (int i = 0; i < k; i++)
         if (c[i]->n1 == n1) return c[i];
       return nullptr;
@@ -225,7 +225,7 @@ extern "C" int qbg_fft_splits(int n, int* n1, int cap) {
   return qbg::guarded(nullptr, [&]() -> int {
     if (!n1 || cap < 0) return QBG_E_INVAL;
     const qbg::F4Ops* c[8];
-    const int k = qbg::f4_candidates(n, c, 8);
+    const int k = qbg::f4_candidates(n, c, 8, true);
     for (int i = 0; i < k && i < cap; i++) n1[i] = c[i]->n1;
     return k;
   });

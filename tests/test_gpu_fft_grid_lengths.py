@@ -120,3 +120,12 @@ def test_fp32_density_rounding(edge, ecut, grid):
     err = np.linalg.norm(rho["fp32"] - rho["fp64"]) / np.linalg.norm(rho["fp64"])
     assert err < 8.0e-8, err
     ctx.close()
+
+
+def test_plans_of_older_builds():
+    """qbg_grid_plan takes every split that a plan may have been written with."""
+    import qbg
+    for n, n1 in ((90, (10, 18)), (96, (12, 16)), (112, (16, 14)), (126, (14, 18)),
+                  (128, (16, 32)), (144, (16, 12)), (160, (16, 20)), (168, (21, 14)),
+                  (198, (18, 22)), (210, (15, 14)), (224, (16, 32))):
+        assert set(n1) <= set(qbg.fft_splits(n)), n
