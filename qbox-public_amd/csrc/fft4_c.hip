@@ -6,7 +6,7 @@ namespace qbg {
 
 static const F4Ops ops_c[] = {
     QBG_F4(12, 12),   // 144
-    QBG_F4(10, 16),   // 160
+    QBG_F4(16, 10),   // 160
     QBG_F4(14, 12),   // 168
 };
 

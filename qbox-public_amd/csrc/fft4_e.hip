@@ -1,5 +1,5 @@
-// fft4_e.hip -- alternative line splits of the lengths 90, 96, 112, 126, 128
-// and 144 (see fft4_kernels.h); the grid's tuner times them against the
+// fft4_e.hip -- alternative line splits of the lengths 90, 112, 126 and 144
+// (see fft4_kernels.h); the grid's tuner times them against the
 // default splits and keeps the faster per axis and precision.
 #include "fft4_kernels.h"
 
@@ -7,10 +7,8 @@ namespace qbg {
 
 static const F4Ops ops_e[] = {
     QBG_F4(9, 10),    // 90
-    QBG_F4(12, 8),    // 96
     QBG_F4(14, 8),    // 112
     QBG_F4(9, 14),    // 126
-    QBG_F4(8, 16),    // 128
     QBG_F4(16, 9),    // 144
 };
 

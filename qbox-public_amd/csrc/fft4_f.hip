@@ -1,13 +1,11 @@
-// fft4_f.hip -- alternative line splits of the lengths 160, 168, 198, 210
-// and 224 (see fft4_kernels.h); the grid's tuner times them against the
+// fft4_f.hip -- alternative line splits of the lengths 198, 210 and 224
+// (see fft4_kernels.h); the grid's tuner times them against the
 // default splits and keeps the faster per axis and precision.
 #include "fft4_kernels.h"
 
 namespace qbg {
 
 static const F4Ops ops_f[] = {
-    QBG_F4(16, 10),   // 160
-    QBG_F4(12, 14),   // 168
     QBG_F4(11, 18),   // 198
     QBG_F4(14, 15),   // 210
     QBG_F4(14, 16),   // 224

@@ -7,10 +7,14 @@ namespace qbg {
 static const F4Ops ops_p[] = {
     QBG_F4(18, 5),    // 90
     QBG_F4(16, 6),    // 96
+    QBG_F4(8, 12),    // 96
     QBG_F4(18, 7),    // 126
     QBG_F4(32, 4),    // 128
+    QBG_F4(8, 16),    // 128
     QBG_F4(20, 8),    // 160
+    QBG_F4(10, 16),   // 160
     QBG_F4(21, 8),    // 168
+    QBG_F4(12, 14),   // 168
     QBG_F4(22, 9),    // 198
     QBG_F4(32, 7),    // 224
 };
