@@ -100,6 +100,11 @@ int qbg_stream_copy(qbg_ctx* ctx, void* dst, const void* src, size_t bytes);
 int qbg_prof_enable(qbg_ctx* ctx, int on);
 int qbg_prof_reset(qbg_ctx* ctx);
 int qbg_prof_read(qbg_ctx* ctx, int kind, double* total_ms, int* count);
+/* How many evaluations of ctx's functionals so far ran their kinetic and
+ * nonlocal part on the context's second stream, beside the transforms: large
+ * ones do, outside captures and while the profiler is off.  The results do
+ * not depend on it.  No counterpart in the reference. */
+int qbg_beside_count(const qbg_ctx* ctx);
 
 /* ------------------------------------------- FourierTransform + mapping */
 /* FourierTransform(const Basis&, np0, np1, np2) with BasisMapping's maps

@@ -67,6 +67,7 @@ qbg::SideScope::SideScope(qbg_ctx* c_) : c(c_), main(c_->stream) {
       hipStreamWaitEvent(c->side, c->fork_ev, 0) != hipSuccess)
     (void)hipStreamSynchronize(main);
   c->stream = c->side;
+  c->beside++;
 }
 
 qbg::SideScope::~SideScope() {
@@ -206,6 +207,8 @@ int qbg_stream_join(qbg_ctx* before, qbg_ctx* after) {
     return QBG_OK;
   });
 }
+
+int qbg_beside_count(const qbg_ctx* c) { return c ? c->beside : 0; }
 
 int qbg_graph_begin(qbg_ctx* c) {
   return qbg::guarded(c, [&]() -> int {

@@ -45,6 +45,7 @@ struct qbg_ctx {
   hipStream_t side = nullptr;
   hipEvent_t fork_ev = nullptr, side_ev = nullptr;
   bool side_pending = false;        // side holds work that stream has not waited for
+  int beside = 0;                   // SideScopes so far (qbg_beside_count)
   bool side_ready();                // creates them at the first use
   void join_side();
   std::string err;

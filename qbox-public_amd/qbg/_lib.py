@@ -58,6 +58,7 @@ SIGNATURES = {
     "qbg_stream_copy": [_vp, _vp, _vp, C.c_size_t],
     "qbg_prof_enable": [_vp, C.c_int],
     "qbg_prof_reset": [_vp],
+    "qbg_beside_count": [_vp],
     "qbg_prof_read": [_vp, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_int)],
     "qbg_gram": [_vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int],
     "qbg_gram_complex": [_vp, _vp, C.c_int, C.c_int, C.c_int],
@@ -221,6 +222,10 @@ class Context:
         d = DArray(self, a.shape, a.dtype)
         d.upload(a)
         return d
+
+    def beside_count(self):
+        """qbg_beside_count: evaluations that used the second stream so far."""
+        return int(self.lib.qbg_beside_count(self.h))
 
     def timer_start(self):
         self.check(self.lib.qbg_timer_start(self.h))
