@@ -690,7 +690,6 @@ static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, do
         (rc = dalloc(c, &e->d_rhogt, (size_t)2 * ngv)) || (rc = dalloc(c, &e->d_vlocal, (size_t)2 * ngv)) ||
         (rc = dalloc(c, &e->d_fesr, 3 * e->nat)) || (rc = dalloc(c, &e->d_fion, 3 * e->nat)) ||
         (rc = dalloc(c, &e->d_scal, S_COUNT)) || (rc = dalloc(c, &e->d_partial, e->partial_doubles)) ||
-        (rc = dalloc(c, &e->d_partial_side, e->partial_doubles)) ||
         (rc = dalloc(c, &e->d_anl, (size_t)2 * e->M * 2 * ngwm)) ||
         (rc = dalloc(c, &e->d_fnl, (size_t)2 * e->M * nst)) ||
         (rc = dalloc(c, &e->d_fout, (size_t)e->M * nst)) ||
@@ -769,8 +768,13 @@ static int ef_create(qbg_ctx* c, const double* cell9, const double* refcell9, do
       delete e;
       return rc;
     }
-    // (here and not at the first evaluation, which may be beside another thread's capture)
-    if ((long)e->ngw_max * nst * nkp >= SIDE_MIN) (void)c->side_ready();
+    // (here and not at the first evaluation, which may be beside another thread's
+    // capture; without its partial sums the functional stays on one stream)
+    if ((long)e->ngw_max * nst * nkp >= SIDE_MIN && c->side_ready() &&
+        hipMalloc((void**)&e->d_partial_side, sizeof(double) * e->partial_doubles) != hipSuccess) {
+      (void)hipGetLastError();
+      e->d_partial_side = nullptr;
+    }
     *out = e;
     return QBG_OK;
   }
@@ -1536,7 +1540,7 @@ static bool ef_side_ok(qbg_ef* e, const double* c, int ldc, int compute_hpsi, co
   const long n = 2L * e->nst * e->nkp;
   if (compute_hpsi && c < hpsi + n * ldh && hpsi < c + n * ldc) return false;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  return ctx->side && hipSetDevice(ctx->device) == hipSuccess &&
+  return ctx->side && e->d_partial_side && hipSetDevice(ctx->device) == hipSuccess &&
          hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess &&
          cap == hipStreamCaptureStatusNone;
 }

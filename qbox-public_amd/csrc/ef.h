@@ -46,7 +46,7 @@ struct qbg_ef {
   double *d_rhor = nullptr, *d_vxc = nullptr, *d_vr = nullptr, *d_rhog = nullptr;
   double *d_rhoelg = nullptr, *d_rhogt = nullptr, *d_vlocal = nullptr, *d_occ = nullptr;
   double *d_fesr = nullptr, *d_fion = nullptr, *d_scal = nullptr, *d_partial = nullptr;
-  double* d_partial_side = nullptr;   // d_partial of work on the side stream
+  double* d_partial_side = nullptr;   // d_partial of work on the side stream, or null
   size_t partial_doubles = 0;
   // nonlocal
   int M = 0;
