@@ -33,7 +33,6 @@ void launch_core_g(int ngv, int nsp, const double* sfac, const double* rhoc, dou
                    double* rhocg, hipStream_t s);
 void launch_core_dxc(int ngv, const double* vxcg, const double* rhocg, double* partial,
                      double* out1, hipStream_t s);
-void launch_lda_points(const double* rho, int n, double* e, double* v, hipStream_t s);
 int launch_vhxc_g(const double* rhog, int ngv, double omega_inv, const double* vion,
                   const double* dvion, const double* rhopst, const double* g2i, const double* gi,
                   const double* gx, double* rhoelg, double* rhogt, double* vlocal, int stress,
@@ -64,9 +63,6 @@ int launch_dmat_enl(const double* F, int M, int nst, const double* occ, const in
                     const int32_t* m_npr, const int32_t* m_stride, const int32_t* m_dbase,
                     const double* dmat, const double* m_wt, double omega_inv, double* fout,
                     const double* occw, double* W, double* partial, hipStream_t s);
-void launch_nl_forces(const double* fout, const double* dF, int M, int nst, const double* occ,
-                      const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
-                      int nat, double* fion, hipStream_t s);
 
 // complex (k != 0) bands on a real band grid (kpoint.hip): each band n of c
 // (on S) to the pair (c1, c2) at columns 2n, 2n+1 of out (on U's half

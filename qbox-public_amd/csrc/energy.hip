@@ -280,15 +280,6 @@ int launch_lsda(const double* rup, const double* rdn, const double* rc, long n, 
   return nb;
 }
 
-// LDA pointwise values for a test vector (no reduction)
-__global__ void k_lda_points(const double* __restrict__ rho, int n, double* e, double* v) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) lda_pz(rho[i], e[i], v[i]);
-}
-void launch_lda_points(const double* rho, int n, double* e, double* v, hipStream_t s) {
-  hipLaunchKernelGGL(k_lda_points, dim3((n + 255) / 256), dim3(256), 0, s, rho, n, e, v);
-}
-
 // ---------------------------------------------------------- vhxc in G
 // src/EnergyFunctional.cpp:243-383: rhoelg = rhog/omega; eps, Hartree sums;
 // rhogt = rhoelg + rhopst; vlocal_g = vion + 4 pi rhogt g2i.
@@ -706,37 +697,6 @@ int launch_dmat_enl(const double* F, int M, int nst, const double* occ, const in
   hipLaunchKernelGGL(k_dmat_enl, dim3(nb), dim3(256), 0, s, F, M, nst, occ, m_ipr, m_npr,
                      m_stride, m_dbase, dmat, m_wt, omega_inv, fout, occw, W, partial);
   return nb;
-}
-
-// fion[3a+j] -= sum_{m of atom a} sum_n 2 occ_n fout[m,n] dF_j[m,n]
-// (src/NonLocalPotential.cpp:1734-1751); one block per (atom, j)
-__global__ __launch_bounds__(256) void k_nl_forces(const double* __restrict__ fout,
-                                                   const double* __restrict__ dF, int M, int nst,
-                                                   const double* __restrict__ occ,
-                                                   const int32_t* __restrict__ a_m0,
-                                                   const int32_t* __restrict__ a_npr,
-                                                   const int32_t* __restrict__ a_stride,
-                                                   double* __restrict__ fion) {
-  // dF is the 3M x nst block of the force GEMM: dF[(j*M + m) + n*3M]
-  const int a = blockIdx.x, j = blockIdx.y;
-  const int m0 = a_m0[a], npr = a_npr[a], st = a_stride[a];
-  double v[1] = {0.0};
-  for (int t = threadIdx.x; t < npr * nst; t += 256) {
-    const int ipr = t % npr, n = t / npr;
-    const int m = m0 + ipr * st;
-    v[0] += 2.0 * occ[n] * fout[(long)n * M + m] * dF[(long)n * 3 * M + (long)j * M + m];
-  }
-  __shared__ double res[1];
-  block_reduce_store<1>(v, res);
-  __syncthreads();
-  if (threadIdx.x == 0) fion[3 * a + j] -= res[0];
-}
-
-void launch_nl_forces(const double* fout, const double* dF, int M, int nst, const double* occ,
-                      const int32_t* a_m0, const int32_t* a_npr, const int32_t* a_stride,
-                      int nat, double* fion, hipStream_t s) {
-  hipLaunchKernelGGL(k_nl_forces, dim3(nat, 3), dim3(256), 0, s, fout, dF, M, nst, occ, a_m0,
-                     a_npr, a_stride, fion);
 }
 
 // Forces by reassociation of src/NonLocalPotential.cpp:1703-1751:

@@ -14,13 +14,6 @@
 namespace qbg {
 namespace f4 {
 
-// factor split chosen for a line length: the divisor pair n1 >= n2 with the
-// smallest n1 (both <= 32); n1 = 0 if none
-__host__ __device__ constexpr int split_n1(int n) {
-  for (int a = 1; a <= 32; a++)
-    if (n % a == 0 && n / a <= a && n / a >= 1) return a;
-  return 0;
-}
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 constexpr int gcd_c(int a, int b) { return b == 0 ? a : gcd_c(b, a % b); }
 // x with a x = 1 (mod m), m > 1, gcd(a, m) = 1

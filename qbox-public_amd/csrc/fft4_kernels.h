@@ -1,6 +1,6 @@
 // fft4_kernels.h -- the five pass kernels with four-step line transforms of
 // compile-time length (N1 x N2), and their launchers.  Instantiated per line
-// length in fft4_sizes.hip; dispatched from fft.hip through f4_ops().
+// length in fft4_a.hip ... fft4_p.hip; dispatched from fft.hip through f4_ops().
 //
 // Workspace layouts (blocked so that every block moves long contiguous
 // runs): zbuf[pair][kb][col][kk] holds plane k = KB*kb + kk of workspace

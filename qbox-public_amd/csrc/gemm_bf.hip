@@ -50,15 +50,6 @@ __device__ __forceinline__ int lds_k(int row, int k) {
   return (((k >> 3) ^ (row >> 1) ^ -((row >> 3) & 1)) & 3) << 3 | (k & 7);
 }
 
-// round-to-nearest-even bfloat16 bits of x; `back` is the value as FP32
-__device__ __forceinline__ unsigned short bf16_rne(float x, float& back) {
-  unsigned u = __float_as_uint(x);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  u &= 0xffff0000u;
-  back = __uint_as_float(u);
-  return (unsigned short)(u >> 16);
-}
-
 // split 8 values into NS parts of 8 bf16 each; the conversions are the
 // hardware's round-to-nearest-even FP32 -> BF16 (packed, two per instruction)
 template <int NS>
