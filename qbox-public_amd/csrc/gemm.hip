@@ -26,9 +26,12 @@
 //     stored), so only the last chunk and the last q tile test anything.
 // 512 bands x 1024 projectors x 461336 in FP64: TN 11.8 -> 8.4 ms (58 TFLOP/s),
 // NN 10.2 -> 7.9 ms (61 TFLOP/s).  Tried and slower or equal: a barrier in the middle of a
-// chunk with the next operands in registers (spills), wave priorities, 96-row
-// tiles.  The tile follows the extents (pick below): the projections
-// of 8 atoms on 16 bands (K = 11364) take 9 us where a 128 x 128 tile took 95.
+// chunk with the next operands in registers (spills), wave priorities.  The tile
+// follows the extents (pick below): the projections of 8 atoms on 16 bands (K = 11364)
+// take 9 us where a 128 x 128 tile took 95.  Tiles of 96 win nothing at that size
+// (512 x 512 x 109 k: 2.87 ms with and without) and 2 to 6 % of the three products
+// where 64 and 128 leave the last tile nearly empty: 90 bands x 288 projectors x 63 k
+// 0.294 -> 0.281 ms in FP64, 0.174 -> 0.165 in FP32, 131 x 300 x 109 k 0.427 -> 0.410 in FP32.
 //
 // MFMA lane layouts on a 64-wide wave (16x16x4): lane l holds A[l%16][l/16]
 // and B[l/16][l%16]; accumulator e of lane l is D[4e + l/16][l%16] for f64
@@ -376,10 +379,10 @@ Pick pick(int np, int nq, long nr, long minS, long maxS, unsigned bjs, int bi_fi
 // The fewest splits of an FP32 product.  A split is one chain of FP32 sums
 // (the splits are added in FP64), whose rounding error grows as the square root
 // of its length, and the cycles alone would halve the splits where two blocks share
-// a CU anyway: 512 bands x 1024 projectors x 461 k in 16 splits, nonlocal H psi off by
-// 2.8e-6; in 32, 1.95e-6, for 1 % more of the product's time (its partials).  So a chain holds at
-// most a 1/32 of the reduction, or, of outputs of more than 32 tiles of 128 x 128, of
-// which 1024 blocks are enough, 1/(1024 / tiles); chains of 64 terms are
+// a CU anyway: 512 bands x 1024 projectors x 461 k in 16 splits leave the nonlocal H psi
+// off by 2.84e-6, in 32 by 1.95e-6, in the same time (31.8 and 31.7 ms an evaluation).
+// So a chain holds at most 1/32 of the reduction; where the output has more than 32
+// tiles of 128 x 128, of which 1024 blocks are enough, 1/(1024 / tiles); and 64 terms are
 // short enough for any.
 long fp32_splits(int np, int nq, long nr) {
   const long tiles = (long)((np + 127) / 128) * ((nq + 127) / 128), chunks = (nr + KC - 1) / KC;

@@ -28,13 +28,14 @@ def ctx():
     c.close()
 
 
-@pytest.mark.parametrize("nst", [1, 2, 31, 32, 33, 63, 65, 96, 97, 128, 129, 161, 257])
-@pytest.mark.parametrize("ngw,shift", [(7, 0), (8, 1), (129, 0), (1500, 1)])
+# (no more bands than the basis spans)
+@pytest.mark.parametrize("nst,ngw,shift",
+                         [(n, g, s) for g, s in ((7, 0), (8, 1), (129, 0), (1500, 1))
+                          for n in (1, 2, 31, 32, 33, 63, 65, 96, 97, 128, 129, 161, 257)
+                          if n <= 2 * g - 1])
 @pytest.mark.parametrize("which", ["gram", "gram_noalloc"])
 def test_gram_ragged(ctx, nst, ngw, shift, which):
     import qbg
-    if 2 * ngw - 1 < nst:
-        pytest.skip("more bands than the basis spans")
     print(f"[case] {which} nst {nst} ngw {ngw} shift {shift}", flush=True)
     rng = np.random.default_rng(nst * 10000 + ngw)
     ldc = ngw + 1
