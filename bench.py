@@ -36,12 +36,13 @@ MFMA_PEAK_TFLOPS = {"fp64": 78.6, "fp32": 157.3, "bf16": 2500.0}
 # for a plain 1 GiB copy (--copy-probe 1024: FETCH_SIZE 0.5 GiB, WRITE_SIZE
 # 1 GiB, so bytes = 1024 (2 FETCH_SIZE + WRITE_SIZE)); commands and the
 # per-kernel figures are in profiles/c3_hbm_traffic.md.  Keyed by workload and
-# precision; "gemm" is the mean of the three projector products of a step.
+# precision; "gemm" is the mean of the three projector products of a step
+# (the projections with the tuner's default plan).
 MEASURED_TRAFFIC = {
     ("c3: 256 atoms L=36 ecut=70Ry 512 bands", "bf16x2"): {
-        "zbwd": 1527706296, "xbwd": 3053536864, "yvmul": 5114448256, "ydens": 2539485224,
-        "xfwd": 3134759020, "zfwd": 2388999046,
-        "gemm": (5263151974 + 3156065408 + 3500000128) // 3,
+        "zbwd": 1527785472, "xbwd": 3053432832, "yvmul": 5117593600, "ydens": 2512644096,
+        "xfwd": 3134744576, "zfwd": 2373312512,
+        "gemm": (4859332608 + 3160444928 + 3511379968) // 3,
     },
 }
 
