@@ -125,8 +125,8 @@ def test_fp32_density_rounding(edge, ecut, grid, bound):
     ctx.close()
 
 
-def test_plans_of_older_builds():
-    """qbg_grid_plan takes every split that a plan may have been written with."""
+def test_splits_of_saved_plans():
+    """qbg_grid_plan takes every split that a plan kept by a caller may name."""
     import qbg
     for n, n1 in ((90, (10, 18)), (96, (12, 16)), (112, (16, 14)), (126, (14, 18)),
                   (128, (16, 32)), (144, (16, 12)), (160, (16, 20)), (168, (21, 14)),
